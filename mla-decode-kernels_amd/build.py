@@ -49,7 +49,7 @@ OBJ_DIR = os.path.join(PKG_DIR, "_build", "obj")  # objects: not shipped to GPU 
 PROBE_LIB = os.path.join(LIB_DIR, "libgqa_stream_probe.so")
 ISSUE_PROBE_LIB = os.path.join(LIB_DIR, "libissue_probe.so")
 HIP_SOURCES = ["gqa_decode_v0.hip", "gqa_decode_split.hip", "gqa_decode_mfma.hip",
-               "gqa_decode_balanced.hip", "mla_decode.hip"]
+               "gqa_decode_balanced.hip", "mla_decode.hip", "mla_decode_wide.hip"]
 # Packed fp32 VALU ops are disabled for all device code.
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",

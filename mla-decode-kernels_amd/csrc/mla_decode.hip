@@ -70,6 +70,9 @@
 // the pieces in order (log-sum-exp), so results are bitwise reproducible.
 #include "gqa_device.hpp"
 #include "gqa_launch.hpp"
+#include "mla_common.hpp"
+#include "mla_plan.hpp"
+#include "mla_wide.hpp"
 #include "mla_decode.h"
 
 #include <algorithm>
@@ -77,26 +80,13 @@
 
 namespace mla {
 
-using gqa::exp2_fast;
-using gqa::f32_to_bf16_bits;
-using gqa::FastDiv;
-using gqa::kLn2;
-using gqa::kLog2e;
-using gqa::kNegInf;
-
-constexpr int kD = MLA_DECODE_HEAD_DIM;     // 576
-constexpr int kDV = MLA_DECODE_HEAD_DIM_V;  // 512
 constexpr int kKSteps = kD / 32;            // 18 QK k-steps
-constexpr int kTile = 32;                   // tokens per tile
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kRowsPerWave = 16;                      // QK^T rows of a wave
 constexpr int kRowsPerGroup = kWaves * kRowsPerWave;  // 128
 constexpr int kRowBlocks = kRowsPerGroup / 16;        // 8 PV row blocks
 constexpr int kTileBlocks = 2 * kKSteps;              // 36 blocks of 1 KiB
-constexpr int kColBlocks = kD / 64;                   // 9 per row block of 8 tokens
-constexpr int kRowBlockBytes = kColBlocks * 1024;
-constexpr int kTileBytes = 4 * kRowBlockBytes;        // 36 KiB
 // Copy instructions per wave per tile: blocks w, w + 8, ...; waves below
 // kWavesHi take one more.
 constexpr int kLoadsHi = (kTileBlocks + kWaves - 1) / kWaves;  // 5
@@ -128,31 +118,6 @@ constexpr int kCopyLo = kCopyWaves == 8 ? kLoadsLo : 0;                // copies
 // checks both operand reads against the measured LDS phase rules above).
 __device__ __forceinline__ int chunk_swz(int rb8, int r) {
   return (int)((0x0052246637751143ull >> (4 * (8 * (rb8 & 1) + r))) & 7u);
-}
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) bf16x4_t lds_bf16x4_t;
-
-struct MlaArgs {
-  const uint16_t* q;
-  const uint16_t* kv;
-  const int* block_table;
-  const int* seq_lens;
-  uint16_t* out;
-  float* lse;
-  float* ws_acc;  // [B, R, ns, 512]
-  float* ws_m;    // [B, R, ns] natural-log units
-  float* ws_l;
-  uint64_t* pre;        // balanced launch: tile prefix sums [B + 2] (written by the split kernel)
-  int B, s_q, h_q, R, block_size, max_blocks, num_splits, causal, nshare;
-  FastDiv bs_div;
-  float scale_log2e;
-};
-
-__device__ __forceinline__ bf16x8_t as_bf16x8(const uint4& u) {
-  return __builtin_bit_cast(bf16x8_t, u);
 }
 
 // A row's probabilities are taken relative to a reference max that is set by
@@ -197,44 +162,6 @@ __device__ unsigned long long mla_phase_cycles[2048][kPhCols];
 #endif
 constexpr int kPAhead = 2;
 
-// Direct HBM -> LDS copies of 16 bytes per lane (global_load_lds_dwordx4):
-// lane x's bytes land at LDS byte address lds + 16 x; lds must be
-// wave-uniform. They are issued through inline assembly so that the compiler
-// does not tie its LDS reads of the other ring slots to these loads'
-// completion (it would wait for every load in flight before each read);
-// completion is awaited explicitly with s_waitcnt vmcnt before the barrier
-// that publishes a tile. The first form addresses base + voff (a uniform
-// 64-bit base, a 32-bit per-lane offset); the second a per-lane address.
-// On gfx9-family GPUs an LDS-DMA instruction needs one wait state after an
-// SALU write of M0; the compiler inserts it for its own LDS-DMA code but does
-// not look inside inline assembly, hence the s_nop (measured cost: up to ~3 %
-// on the matrix-bound s_q = 2 workloads).
-// M0 is a register the compiler reserves (hipcc notes the clobber as such and
-// will not restore it): these kernels rely on the compiler emitting no M0 use
-// of its own, which tests/test_mla_codegen.py checks on the generated code,
-// together with the spill-free and wait-free tile loops.
-__device__ __forceinline__ void load_to_lds(const uint16_t* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-               :
-               : "v"(voff), "s"(base), "s"(lds)
-               : "memory", "m0");
-}
-__device__ __forceinline__ void load_to_lds(const uint16_t* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-               :
-               : "v"(src), "s"(lds)
-               : "memory", "m0");
-}
-
-// Waits until at most kInFlight of this wave's direct loads are outstanding
-// (they complete in issue order) and its LDS writes are done, then joins the
-// workgroup barrier; LDS reads and writes are not moved across it.
-template <int kInFlight>
-__device__ __forceinline__ void publish_barrier() {
-  static_assert(kInFlight >= 0 && kInFlight < 64, "vmcnt holds 6 bits");
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(kInFlight) : "memory");
-}
-
 // Max over lanes l, l ^ 16, l ^ 32 and l ^ 48, the four lanes that hold one
 // row in the MFMA C layout: v_permlane16_swap (v_permlane32_swap) with both
 // operands x hands every lane x of itself and of its xor-16 (xor-32) partner,
@@ -253,46 +180,11 @@ __device__ __forceinline__ float row_max(float x) {
   return fmaxf(__uint_as_float(b0), __uint_as_float(b1));
 }
 
-// Where a piece's results go: normalised rows to out and lse (direct), or
-// unnormalised states, row r of the piece's request at index
-// st_base + r * st_stride of ws_acc (x 512), ws_m and ws_l.
-struct PieceOut {
-  bool direct;
-  size_t st_base;
-  int st_stride;
-};
-
 // After a pass, P buffer 1 (first written in the second interval of a pass,
 // two barriers after any pass starts) holds the restart votes and the rows'
 // final sums.
 constexpr int kStatL = 0;    // 128 floats: row sums
 constexpr int kVotes = 512;  // 8 ints
-
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) u32x4_t lds_u32x4_t;
-typedef __attribute__((address_space(3))) u32x2_t lds_u32x2_t;
-
-// LDS accesses by 32-bit LDS byte address.
-__device__ __forceinline__ u32x4_t lds_load16(uint32_t addr) {
-  return *(const lds_u32x4_t*)(uintptr_t)addr;
-}
-__device__ __forceinline__ void lds_store8(uint32_t addr, u32x2_t v) {
-  *(lds_u32x2_t*)(uintptr_t)addr = v;
-}
-__device__ __forceinline__ bf16x4_t lds_load_tr(uint32_t addr) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4_t*)(uintptr_t)addr);
-}
-__device__ __forceinline__ bf16x8_t as_bf16x8(const u32x4_t& u) {
-  return __builtin_bit_cast(bf16x8_t, u);
-}
-
-// Hands x back through an empty asm statement, so that the compiler treats it
-// as a new value: applied to the lane's operand offsets at the top of every
-// interval, it keeps values derived from them (offset ^ constant, one per
-// matrix step) from being hoisted out of the tile loop, where they would
-// outgrow the register budget of two waves per SIMD.
-__device__ __forceinline__ void refresh(uint32_t& x) { asm volatile("" : "+v"(x)); }
 
 // The workgroup's 128 query rows (row group rg) of request b against tokens
 // [seg_start, seg_end) of the request's S live tokens. Every wave of the
@@ -853,11 +745,6 @@ __global__ __launch_bounds__(256) void mla_decode_merge_kernel(const MlaArgs a) 
 // than shares, only the first T shares take work (one tile each), so every
 // working share is non-empty.
 
-// Share w's first tile.
-__device__ __forceinline__ uint64_t share_start(uint64_t T, int w, int n) {
-  return (uint64_t)w * T / (uint64_t)n;
-}
-
 // Workgroup (w, rg): share w of row group rg. Every workgroup first plans
 // the launch itself from seq_lens (no separate plan launch): the tile counts'
 // inclusive prefix sums over chunks of the batch (one chunk per thread, a
@@ -965,12 +852,12 @@ __global__ __launch_bounds__(256) void mla_decode_balanced_merge_kernel(const Ml
     }
     return;
   }
-  // Shares holding tile p0 and tile p1 - 1: the largest w with start(w) <= t.
-  const int w_lo = (int)(((p0 + 1) * (uint64_t)n - 1) / T);
-  const int w_hi = (int)((p1 * (uint64_t)n - 1) / T);
+  // Shares holding the request's first and last tile.
+  const int w_lo = share_of(T, p0 + (uint64_t)a.piece_cost, n);
+  const int w_hi = share_of(T, p1 - 1, n);
   if (w_lo == w_hi) return;
-  // Pieces: share w_lo's last slot (its first if the request starts the
-  // share), then the first slot of each later share up to w_hi.
+  // Pieces: share w_lo's last slot (its first if no earlier request has tiles
+  // there), then the first slot of each later share up to w_hi.
   const int first_slot = 2 * w_lo + (p0 > share_start(T, w_lo, n) ? 1 : 0);
   merge_row(a, br, w_hi - w_lo + 1, [&](int i) {
     return (size_t)(i == 0 ? first_slot : 2 * (w_lo + i)) * a.R + row;
@@ -1024,6 +911,7 @@ hipError_t make_args(mla::MlaArgs* a, const uint16_t* q, const uint16_t* kv_cach
   a->ws_acc = a->ws_m = a->ws_l = nullptr;
   a->pre = nullptr;
   a->nshare = 0;
+  a->piece_cost = 0;
   a->s_q = s_q;
   a->h_q = h_q;
   a->R = (int)R;
@@ -1046,6 +934,7 @@ hipError_t make_args(mla::MlaArgs* a, const uint16_t* q, const uint16_t* kv_cach
 }
 
 hipError_t launch_splitkv(const mla::MlaArgs& a, hipStream_t stream) {
+  if (mla::wide_splitkv(a)) return mla::launch_wide_splitkv(a, stream);
   const dim3 grid((unsigned)((a.R + mla::kRowsPerGroup - 1) / mla::kRowsPerGroup), a.B,
                   a.num_splits);
   if (a.block_size % mla::kTile == 0)
@@ -1059,6 +948,13 @@ hipError_t launch_combine(const mla::MlaArgs& a, hipStream_t stream) {
   const size_t rows = (size_t)a.B * a.R;
   hipLaunchKernelGGL(mla::mla_decode_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
                      stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_balanced_merge(const mla::MlaArgs& a, hipStream_t stream) {
+  const size_t rows = (size_t)a.B * a.R;
+  hipLaunchKernelGGL(mla::mla_decode_balanced_merge_kernel, dim3((unsigned)((rows + 3) / 4)),
+                     dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -1155,6 +1051,11 @@ extern "C" int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_
   a.pre = reinterpret_cast<uint64_t*>(ws + align16(states * (mla::kDV + 2) * sizeof(float)));
   a.nshare = n;
   const unsigned rg = (unsigned)((a.R + mla::kRowsPerGroup - 1) / mla::kRowsPerGroup);
+  if (mla::wide_balanced(a)) {
+    a.piece_cost = mla::kWidePieceCost;
+    if ((err = mla::launch_wide_balanced(a, stream)) != hipSuccess) return err;
+    return launch_balanced_merge(a, stream);
+  }
   if (block_size % mla::kTile == 0)
     hipLaunchKernelGGL(mla::mla_decode_balanced_kernel<true>, dim3(n, rg), dim3(mla::kThreads), 0,
                        stream, a);
@@ -1162,12 +1063,8 @@ extern "C" int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_
     hipLaunchKernelGGL(mla::mla_decode_balanced_kernel<false>, dim3(n, rg), dim3(mla::kThreads), 0,
                        stream, a);
   if ((err = hipGetLastError()) != hipSuccess) return err;
-  const size_t rows = (size_t)B * a.R;
-  hipLaunchKernelGGL(mla::mla_decode_balanced_merge_kernel, dim3((unsigned)((rows + 3) / 4)),
-                     dim3(256), 0, stream, a);
-  return hipGetLastError();
+  return launch_balanced_merge(a, stream);
 }
-
 
 #if MLA_PHASE_TIMING
 // Profiling build only (not part of include/mla_decode.h): copies the phase

@@ -74,8 +74,10 @@ def get_mla_metadata(cache_seqlens, num_heads_per_head_k, num_heads_k=1, max_seq
     groups = max(1, -(-rows // 128))
     nwg = cus or 256
     meta[0, 1] = nwg
-    # Pieces per request under the balanced plan (share w of n takes tiles
-    # [w T / n, (w + 1) T / n) of the request-ordered 32-token tiles).
+    # Pieces per request with the request-ordered 32-token tiles cut into equal
+    # shares (share w of n: tiles [w T / n, (w + 1) T / n)). The launch plans
+    # for itself on the device and also weighs what a request costs besides its
+    # tiles, so it may cut a request once more or less than reported here.
     n_share = max(1, nwg // groups)
     tiles = (cache_seqlens.clamp(min=0).to(torch.int64) + 31) // 32
     pre = torch.cumsum(tiles, 0)

@@ -22,7 +22,8 @@ REPO_ROOT = os.path.dirname(PKG_DIR)
 SOURCES = {
     "gqa": ["mla-decode-kernels_amd/csrc/gqa_*.hip", "mla-decode-kernels_amd/csrc/gqa_*.hpp",
             "include/gqa_decode.h", "mla-decode-kernels_amd/python/gqa_decode_ext.cpp"],
-    "mla": ["mla-decode-kernels_amd/csrc/mla_decode.hip", "include/mla_decode.h",
+    "mla": ["mla-decode-kernels_amd/csrc/mla_*.hip", "mla-decode-kernels_amd/csrc/mla_*.hpp",
+            "include/mla_decode.h",
             "mla-decode-kernels_amd/python/mla.py"],
 }
 

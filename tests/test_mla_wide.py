@@ -1,0 +1,138 @@
+"""The one-wave-per-SIMD MLA kernels (csrc/mla_decode_wide.hip): GPU parity with
+the oracle at the sizes where they can go wrong -- row counts around the 16, 32,
+64 and 128 rows of their variants, pieces around one, two and three tiles (their
+ring holds four), shares of many short pieces, second passes in the middle of a
+share -- and CPU checks of the generated code.
+
+Tolerance (that of test_mla.py): weights are rounded to bf16 for the PV product
+and the output to bf16, each within 2^-9 relative, so |out - oracle| is at most
+2^-8 of the largest value row entry (~4.5 for N(0, 1)): 1.8e-2.
+"""
+
+import os
+import re
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+import torch
+
+from cases import make_mla_case
+from test_mla import SCALE, check, oracle, run, run_balanced
+from test_mla_codegen import HIPCC, ROOT, kernel_body, tile_loops
+
+EDGES = [1, 31, 32, 33, 0, 63, 64, 65, 95, 96, 97, 128, 129, 161, 300]
+# (s_q, h_q): one row; the 16-, 32-, 64- and 128-row variants, full and one
+# short or over; a second row group.
+ROWS = [(1, 1), (1, 15), (1, 16), (1, 17), (2, 16), (1, 33), (4, 16), (1, 65), (1, 97), (2, 64),
+        (1, 129)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s_q,h_q", ROWS)
+@pytest.mark.parametrize("bs", [32, 64, 96])
+def test_rows_and_tile_edges(gpu, s_q, h_q, bs):
+    print(f"wide s_q={s_q} h_q={h_q} bs={bs}", flush=True)
+    case = make_mla_case(EDGES, s_q, h_q, bs, pool_factor=1.5, seed=h_q + bs, device="cuda",
+                         poison=True)
+    for causal in {False, s_q > 1}:
+        want = oracle(case, causal)
+        for nwg in (1, 3, 40, 256):  # one share of every piece ... one tile per share
+            check(run_balanced(case, causal, nwg), want, f"bal n{nwg}/c{causal}")
+        for ns in (1, 2, 7):
+            check(run(case, causal, ns), want, f"ns{ns}/c{causal}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s_q,h_q", [(1, 16), (1, 32), (1, 64), (1, 128)])
+def test_second_pass_mid_share(gpu, s_q, h_q):
+    # Keys that beat everything else by more than 128 log2 units (fp32 overflows
+    # without the second pass), past their piece's first tile, in pieces that
+    # follow and precede others of the same share.
+    S_list = [40, 700, 33, 300, 95]
+    case = make_mla_case(S_list, s_q, h_q, 64, pool_factor=1.5, seed=7, device="cuda", poison=True)
+    q, kv, bt, sl = case
+    for b, row, tok in ((1, h_q - 1, 405), (1, h_q // 2, 690), (3, 1, 45), (4, 5, 94)):
+        kv[int(bt[b, tok // 64]), tok % 64, 0] = (q[b, 0, row].float() * 5).to(torch.bfloat16)
+        ids = bt[b, :-(-S_list[b] // 64)].long()
+        keys = kv[ids].flatten(0, 1)[:S_list[b], 0].double().cpu()
+        sc = (keys @ q[b, 0, row].double().cpu()).numpy() * SCALE / np.log(2.0)
+        assert sc[tok] - np.delete(sc, tok).max() > 128.0
+    want = oracle(case, False)
+    for nwg in (1, 2, 5):
+        got = run_balanced(case, False, nwg)
+        assert torch.isfinite(got[0].float()).all()
+        check(got, want, f"h{h_q}/n{nwg}")
+    for ns in (1, 3):
+        check(run(case, False, ns), want, f"h{h_q}/ns{ns}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,ns", [(4096, 2), (4160, 2), (256, 1), (320, 1)])
+def test_either_side_of_the_rules(gpu, S, ns):
+    # 2048 tokens per split, 8 tiles in all: either side runs another kernel.
+    case = make_mla_case([S], 1, 128, 64, seed=S, device="cuda")
+    want = oracle(case, False)
+    check(run(case, False, ns), want, f"S{S}/ns{ns}")
+    check(run_balanced(case, False, 256), want, f"S{S}/bal")
+
+
+@pytest.fixture(scope="module")
+def asm(tmp_path_factory):
+    if not shutil.which(HIPCC):
+        pytest.skip("hipcc not available")
+    out = tmp_path_factory.mktemp("mla_wide") / "wide.s"
+    csrc = os.path.join(ROOT, "mla-decode-kernels_amd", "csrc")
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang",
+                    "-target-feature", "-Xclang", "-packed-fp32-ops", "--cuda-device-only", "-S",
+                    f"-I{os.path.join(ROOT, 'include')}", f"-I{csrc}",
+                    os.path.join(csrc, "mla_decode_wide.hip"), "-o", str(out)], check=True,
+                   capture_output=True)
+    return out.read_text()
+
+
+def vgprs(text):
+    """The VGPR numbers named in an operand list."""
+    regs = set()
+    for lo, hi in re.findall(r"\bv\[(\d+):(\d+)\]", text):
+        regs.update(range(int(lo), int(hi) + 1))
+    regs.update(int(x) for x in re.findall(r"\bv(\d+)\b", text))
+    return regs
+
+
+@pytest.mark.parametrize("kernel", ["15mla_wide_kernel", "24mla_wide_balanced_kernel"])
+@pytest.mark.parametrize("rw,m,mfmas", [(32, 4, 68), (16, 4, 68), (16, 2, 52), (16, 1, 44)])
+def test_generated_tile_loop(asm, kernel, rw, m, mfmas):
+    name = f"_ZN3mla12_GLOBAL__N_1{kernel}ILi{rw}ELi{m}EEEvNS_7MlaArgsE"
+    body = kernel_body(asm, name)
+    # M0 belongs to the copies (inline assembly) alone.
+    assert not re.search(r"\bm0\b", re.sub(r";;#ASMSTART.*?;;#ASMEND", "", body, flags=re.S))
+    # (The loop over pieces holds the prologue's QK^T as well; the tile loop is
+    # the innermost loop that issues MFMAs.)
+    shape = "v_mfma_f32_32x32x16_bf16" if rw == 32 else "v_mfma_f32_16x16x32_bf16"
+    loops = [t for t in tile_loops(body) if t.count(shape) == mfmas]
+    assert len(loops) == 1, "tile loop not found"
+    text = loops[0]
+    code = [ln for ln in text.split("\n") if ln.strip() and not ln.strip().startswith(";")]
+    assert not [ln for ln in code if "scratch_" in ln], "spill access inside the tile loop"
+    assert not [ln for ln in code if "v_accvgpr" in ln], "accumulators copied inside the tile loop"
+    own = re.sub(r";;#ASMSTART.*?(;;#ASMEND|\Z)", "", text, flags=re.S)
+    assert "vmcnt" not in own, "compiler vmcnt wait inside the tile loop"
+    # The QK^T results (MFMAs in inline assembly, whose latency the compiler
+    # does not know) are not touched before three more MFMAs have issued.
+    ops = [ln.split(";")[0].strip() for ln in code]
+    qk = [i for i, op in enumerate(ops) if op.startswith(shape + " v[")]
+    assert len(qk) == 36
+    dst = set()
+    for i in qk[-4:]:
+        dst |= vgprs(ops[i].split(",")[0])
+    later = 0
+    for op in ops[qk[-1] + 1:]:
+        if op.startswith("v_mfma"):
+            later += 1
+            if later == 3:
+                break
+        elif op.startswith(("v_", "ds_", "global_", "buffer_")):
+            assert not vgprs(op) & dst, f"QK^T result touched too early: {op}"
+    assert later == 3
