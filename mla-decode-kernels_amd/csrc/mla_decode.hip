@@ -673,63 +673,128 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_kernel(const MlaArgs a
   mla_piece<kBlockUniform>(a, smem, b, blockIdx.x, S, seg_start, seg_end, po);
 }
 
-// Log-sum-exp fold of `count` states of one (request, query row), in order,
-// into out and lse: one wave per row, lane i owns dims 8i .. 8i + 8. index(i)
-// is the state index of the i-th; states with m = -inf (no key) add nothing.
-template <typename IndexFn>
-__device__ __forceinline__ void merge_row(const MlaArgs& a, size_t br, int count, IndexFn index) {
-  constexpr int kBatch = 8;
+// The merges: log-sum-exp folds of the `count` states of each query row of a
+// request into out and lse. A lane owns dims 8 i .. 8 i + 8; a state with m =
+// -inf (no key) adds nothing, the factor of the state holding the max is
+// exactly 1.
+struct RowSum {
+  float L, A[8];
+};
+
+// States first, first + step, ... of a row's `count` (state indices from
+// index(i)) relative to the row's max M, in order, kBatch loaded together.
+template <int kBatch, typename IndexFn>
+__device__ __forceinline__ RowSum fold_states(const MlaArgs& a, float M, int first, int step,
+                                              int count, IndexFn index) {
   const int lane = threadIdx.x & 63;
-  float mloc = kNegInf;
-  for (int i = lane; i < count; i += 64) mloc = fmaxf(mloc, a.ws_m[index(i)]);
-  const float M = gqa::wave_max(mloc);
-  float L = 0.f, A[8];
+  RowSum s;
+  s.L = 0.f;
 #pragma unroll
-  for (int d = 0; d < 8; ++d) A[d] = 0.f;
-  if (M != kNegInf) {
-    for (int i0 = 0; i0 < count; i0 += kBatch) {
-      float mi[kBatch], li[kBatch];
-      float4 a0[kBatch], a1[kBatch];
+  for (int d = 0; d < 8; ++d) s.A[d] = 0.f;
+  for (int i0 = first; i0 < count; i0 += kBatch * step) {
+    float mi[kBatch], li[kBatch];
+    float4 a0[kBatch], a1[kBatch];
 #pragma unroll
-      for (int k = 0; k < kBatch; ++k) {
-        const size_t sx = index(min(i0 + k, count - 1));  // past the end: valid, not folded
-        mi[k] = a.ws_m[sx];
-        li[k] = a.ws_l[sx];
-        const float4* src = reinterpret_cast<const float4*>(a.ws_acc + sx * kDV + 8 * lane);
-        a0[k] = src[0];
-        a1[k] = src[1];
-      }
+    for (int k = 0; k < kBatch; ++k) {
+      if (k > 0 && i0 + k * step >= count) break;  // (uniform)
+      const size_t sx = index(i0 + k * step);
+      mi[k] = a.ws_m[sx];
+      li[k] = a.ws_l[sx];
+      const float4* src = reinterpret_cast<const float4*>(a.ws_acc + sx * kDV + 8 * lane);
+      a0[k] = src[0];
+      a1[k] = src[1];
+    }
 #pragma unroll
-      for (int k = 0; k < kBatch; ++k) {
-        if (i0 + k >= count) break;
-        // Exactly 1 for the state holding the max; 0 for empty states.
-        const float f = mi[k] == M ? 1.f : exp2_fast((mi[k] - M) * kLog2e);
-        const float av[8] = {a0[k].x, a0[k].y, a0[k].z, a0[k].w, a1[k].x, a1[k].y, a1[k].z, a1[k].w};
-        L = fmaf(li[k], f, L);
+    for (int k = 0; k < kBatch; ++k) {
+      if (k > 0 && i0 + k * step >= count) break;
+      const float f = mi[k] == M ? 1.f : exp2_fast((mi[k] - M) * kLog2e);
+      const float av[8] = {a0[k].x, a0[k].y, a0[k].z, a0[k].w, a1[k].x, a1[k].y, a1[k].z, a1[k].w};
+      s.L = fmaf(li[k], f, s.L);
 #pragma unroll
-        for (int d = 0; d < 8; ++d) A[d] = fmaf(av[d], f, A[d]);
-      }
+      for (int d = 0; d < 8; ++d) s.A[d] = fmaf(av[d], f, s.A[d]);
     }
   }
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  return s;
+}
+
+template <typename IndexFn>
+__device__ __forceinline__ float max_of_states(const MlaArgs& a, int count, IndexFn index) {
+  float m = kNegInf;
+  for (int i = threadIdx.x & 63; i < count; i += 64) m = fmaxf(m, a.ws_m[index(i)]);
+  return gqa::wave_max(m);
+}
+
+__device__ __forceinline__ void store_row(const MlaArgs& a, int b, int row, float M,
+                                          const RowSum& s) {
+  const int lane = threadIdx.x & 63;
+  const float inv = s.L > 0.f ? 1.f / s.L : 0.f;
   uint32_t wv[4];
 #pragma unroll
   for (int d = 0; d < 4; ++d)
-    wv[d] = f32_to_bf16_bits(A[2 * d] * inv) | (f32_to_bf16_bits(A[2 * d + 1] * inv) << 16);
-  *reinterpret_cast<uint4*>(a.out + br * kDV + 8 * lane) = make_uint4(wv[0], wv[1], wv[2], wv[3]);
+    wv[d] = f32_to_bf16_bits(s.A[2 * d] * inv) | (f32_to_bf16_bits(s.A[2 * d + 1] * inv) << 16);
+  *reinterpret_cast<uint4*>(a.out + ((size_t)b * a.R + row) * kDV + 8 * lane) =
+      make_uint4(wv[0], wv[1], wv[2], wv[3]);
   if (a.lse && lane == 0) {
-    const int b = (int)(br / a.R), row = (int)(br - (size_t)b * a.R);
     const int qi = row / a.h_q, h = row - qi * a.h_q;
-    a.lse[((size_t)b * a.h_q + h) * a.s_q + qi] = L > 0.f ? M + logf(L) : kNegInf;
+    a.lse[((size_t)b * a.h_q + h) * a.s_q + qi] = s.L > 0.f ? M + logf(s.L) : kNegInf;
   }
 }
 
-// Fixed splits: the num_splits states of each row, in split order.
-__global__ __launch_bounds__(256) void mla_decode_merge_kernel(const MlaArgs a) {
-  const size_t br = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (br >= (size_t)a.B * a.R) return;
-  const int ns = a.num_splits;
-  merge_row(a, br, ns, [&](int i) { return br * ns + i; });
+// One workgroup of NW waves merges rows r0 .. r0 + RPW - 1 of request b, each
+// from `count` states (index(row, i)). Few states: a wave per row, in order.
+// Many: all waves share each row, wave w taking states w, w + NW, ..., and the
+// waves' sums are added in wave order. Either way the order is fixed by the
+// launch, so results are bitwise reproducible.
+template <int NW, int RPW, typename IndexFn>
+__device__ __forceinline__ void merge_rows(const MlaArgs& a, int b, int r0, int count,
+                                           IndexFn index) {
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  if (RPW == NW && count <= 4 * NW) {
+    const int row = r0 + wv;
+    if (row >= a.R) return;
+    const float M = max_of_states(a, count, [&](int i) { return index(row, i); });
+    RowSum s = {};
+    if (M != kNegInf)
+      s = fold_states<8>(a, M, 0, 1, count, [&](int i) { return index(row, i); });
+    store_row(a, b, row, M, s);
+    return;
+  }
+  __shared__ float part[NW][kDV + 64];  // a wave's A (lane-major), then its L
+  const int rows = min(RPW, a.R - r0);
+  for (int k = 0; k < rows; ++k) {
+    const int row = r0 + k;
+    const float M = max_of_states(a, count, [&](int i) { return index(row, i); });
+    RowSum s = {};
+    if (M != kNegInf)
+      s = fold_states<8>(a, M, wv, NW, count, [&](int i) { return index(row, i); });
+    if (k > 0) __syncthreads();
+    reinterpret_cast<float4*>(part[wv])[2 * lane] = make_float4(s.A[0], s.A[1], s.A[2], s.A[3]);
+    reinterpret_cast<float4*>(part[wv])[2 * lane + 1] = make_float4(s.A[4], s.A[5], s.A[6], s.A[7]);
+    if (lane == 0) part[wv][kDV] = s.L;
+    __syncthreads();
+    if (wv == 0) {
+      RowSum t = {};
+#pragma unroll
+      for (int x = 0; x < NW; ++x) {
+        const float4 v0 = reinterpret_cast<const float4*>(part[x])[2 * lane];
+        const float4 v1 = reinterpret_cast<const float4*>(part[x])[2 * lane + 1];
+        const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        t.L += part[x][kDV];
+#pragma unroll
+        for (int d = 0; d < 8; ++d) t.A[d] += v[d];
+      }
+      store_row(a, b, row, M, t);
+    }
+  }
+}
+
+// Fixed splits: the num_splits states of each row.
+template <int NW, int RPW>
+__global__ __launch_bounds__(64 * NW) void mla_decode_merge_kernel(const MlaArgs a) {
+  const int b = blockIdx.y, ns = a.num_splits;
+  merge_rows<NW, RPW>(a, b, blockIdx.x * RPW, ns,
+                      [&](int row, int i) { return ((size_t)b * a.R + row) * ns + i; });
 }
 
 // ---------------------------------------------------------------------------
@@ -837,29 +902,27 @@ __global__ __launch_bounds__(kThreads, 1) void mla_decode_balanced_kernel(const 
 // Rows of requests cut by share boundaries: fold their pieces in share order
 // (shares with no tiles hold no piece). Requests with no tiles get out = 0 and
 // lse = -inf; whole pieces were written by the decode kernel.
-__global__ __launch_bounds__(256) void mla_decode_balanced_merge_kernel(const MlaArgs a) {
-  const size_t br = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (br >= (size_t)a.B * a.R) return;
-  const int b = (int)(br / a.R), row = (int)(br - (size_t)b * a.R);
-  const uint64_t p0 = a.pre[b], p1 = a.pre[b + 1], T = a.pre[a.B];
-  const int n = (int)a.pre[a.B + 1];
+template <int NW, int RPW>
+__global__ __launch_bounds__(64 * NW) void mla_decode_balanced_merge_kernel(const MlaArgs a) {
+  const int b = blockIdx.y, r0 = blockIdx.x * RPW;
+  // Written by the split kernel; read-only here (the uniform loads are scalar).
+  const __attribute__((address_space(4))) uint64_t* pre =
+      (const __attribute__((address_space(4))) uint64_t*)a.pre;
+  const uint64_t p0 = pre[b], p1 = pre[b + 1], U = pre[a.B];
+  const int n = (int)pre[a.B + 1];
   if (p1 == p0) {
-    const int lane = threadIdx.x & 63;
-    *reinterpret_cast<uint4*>(a.out + br * kDV + 8 * lane) = make_uint4(0, 0, 0, 0);
-    if (a.lse && lane == 0) {
-      const int qi = row / a.h_q, h = row - qi * a.h_q;
-      a.lse[((size_t)b * a.h_q + h) * a.s_q + qi] = kNegInf;
-    }
+    const int row = r0 + (int)(threadIdx.x >> 6);
+    if (threadIdx.x < 64 * RPW && row < a.R) store_row(a, b, row, kNegInf, RowSum{});
     return;
   }
   // Shares holding the request's first and last tile.
-  const int w_lo = share_of(T, p0 + (uint64_t)a.piece_cost, n);
-  const int w_hi = share_of(T, p1 - 1, n);
+  const int w_lo = share_of(U, p0 + (uint64_t)a.piece_cost, n);
+  const int w_hi = share_of(U, p1 - 1, n);
   if (w_lo == w_hi) return;
   // Pieces: share w_lo's last slot (its first if no earlier request has tiles
   // there), then the first slot of each later share up to w_hi.
-  const int first_slot = 2 * w_lo + (p0 > share_start(T, w_lo, n) ? 1 : 0);
-  merge_row(a, br, w_hi - w_lo + 1, [&](int i) {
+  const int first_slot = 2 * w_lo + (p0 > share_start(U, w_lo, n) ? 1 : 0);
+  merge_rows<NW, RPW>(a, b, r0, w_hi - w_lo + 1, [&](int row, int i) {
     return (size_t)(i == 0 ? first_slot : 2 * (w_lo + i)) * a.R + row;
   });
 }
@@ -944,17 +1007,35 @@ hipError_t launch_splitkv(const mla::MlaArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// Rows of up to `pieces` states each: one row per workgroup of 16 waves where
+// rows are few and pieces many, else 4 rows per workgroup of 4 waves. One
+// request of 4096 tokens and 128 rows at 128 pieces: the fold alone took 51.7
+// us with a wave per row (32 workgroups, 16 round trips each). At 512 rows
+// (4 requests of 256 to 1024 tokens) 16 waves per row lose 10-20 % of the step
+// to 4, at 1024 rows up to a third.
+bool merge_wide(const mla::MlaArgs& a, int64_t pieces) {
+  return pieces >= 16 && (int64_t)a.B * a.R <= 256;
+}
+
 hipError_t launch_combine(const mla::MlaArgs& a, hipStream_t stream) {
-  const size_t rows = (size_t)a.B * a.R;
-  hipLaunchKernelGGL(mla::mla_decode_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0,
-                     stream, a);
+  if (merge_wide(a, a.num_splits))
+    hipLaunchKernelGGL((mla::mla_decode_merge_kernel<16, 1>), dim3(a.R, a.B), dim3(1024), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((mla::mla_decode_merge_kernel<4, 4>), dim3((a.R + 3) / 4, a.B), dim3(256),
+                       0, stream, a);
   return hipGetLastError();
 }
 
 hipError_t launch_balanced_merge(const mla::MlaArgs& a, hipStream_t stream) {
-  const size_t rows = (size_t)a.B * a.R;
-  hipLaunchKernelGGL(mla::mla_decode_balanced_merge_kernel, dim3((unsigned)((rows + 3) / 4)),
-                     dim3(256), 0, stream, a);
+  // A request has at most its share of the shares, and one piece per tile.
+  const int64_t tiles = ((int64_t)a.max_blocks * a.block_size + mla::kTile - 1) / mla::kTile;
+  if (merge_wide(a, std::min<int64_t>(a.nshare / a.B, tiles)))
+    hipLaunchKernelGGL((mla::mla_decode_balanced_merge_kernel<16, 1>), dim3(a.R, a.B), dim3(1024),
+                       0, stream, a);
+  else
+    hipLaunchKernelGGL((mla::mla_decode_balanced_merge_kernel<4, 4>), dim3((a.R + 3) / 4, a.B),
+                       dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

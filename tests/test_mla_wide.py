@@ -136,3 +136,22 @@ def test_generated_tile_loop(asm, kernel, rw, m, mfmas):
         elif op.startswith(("v_", "ds_", "global_", "buffer_")):
             assert not vgprs(op) & dst, f"QK^T result touched too early: {op}"
     assert later == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s_q,h_q", [(1, 5), (1, 128), (2, 100), (2, 128), (3, 128)])
+@pytest.mark.parametrize("S_list", [[511], [512], [4096], [9000, 40], [2000, 1, 0, 700]])
+def test_merges(gpu, s_q, h_q, S_list):
+    # Rows of few and of many pieces (from 16 on, up to 256 rows: 16 waves a
+    # row; else a wave a row up to 16 pieces, 4 waves beyond), rows off the four
+    # of a workgroup, and requests that are not cut at all.
+    case = make_mla_case(S_list, s_q, h_q, 64, pool_factor=1.5, seed=h_q, device="cuda",
+                         poison=True)
+    want = oracle(case, False)
+    for nwg in (40, 256):
+        first = run_balanced(case, False, nwg)
+        check(first, want, f"bal n{nwg}")
+        again = run_balanced(case, False, nwg)
+        assert torch.equal(first[0], again[0]) and torch.equal(first[1], again[1])
+    for ns in (3, 15, 16, 17, 64):
+        check(run(case, False, ns), want, f"ns{ns}")
