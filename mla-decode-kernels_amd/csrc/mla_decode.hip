@@ -741,52 +741,42 @@ __device__ __forceinline__ void store_row(const MlaArgs& a, int b, int row, floa
 }
 
 // One workgroup of NW waves merges rows r0 .. r0 + RPW - 1 of request b, each
-// from `count` states (index(row, i)). Few states: a wave per row, in order.
-// Many: all waves share each row, wave w taking states w, w + NW, ..., and the
-// waves' sums are added in wave order. Either way the order is fixed by the
-// launch, so results are bitwise reproducible.
+// from `count` states (index(row, i)). RPW == NW: a wave per row, in order.
+// RPW == 1: all waves share the row, wave w taking states w, w + NW, ..., and
+// the waves' sums are added in wave order. Either way the order is fixed by
+// the launch, so results are bitwise reproducible.
 template <int NW, int RPW, typename IndexFn>
 __device__ __forceinline__ void merge_rows(const MlaArgs& a, int b, int r0, int count,
                                            IndexFn index) {
+  static_assert(RPW == NW || RPW == 1);
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int lane = threadIdx.x & 63;
-  if (RPW == NW && count <= 4 * NW) {
-    const int row = r0 + wv;
-    if (row >= a.R) return;
-    const float M = max_of_states(a, count, [&](int i) { return index(row, i); });
-    RowSum s = {};
-    if (M != kNegInf)
-      s = fold_states<8>(a, M, 0, 1, count, [&](int i) { return index(row, i); });
-    store_row(a, b, row, M, s);
-    return;
-  }
-  __shared__ float part[NW][kDV + 64];  // a wave's A (lane-major), then its L
-  const int rows = min(RPW, a.R - r0);
-  for (int k = 0; k < rows; ++k) {
-    const int row = r0 + k;
-    const float M = max_of_states(a, count, [&](int i) { return index(row, i); });
-    RowSum s = {};
-    if (M != kNegInf)
-      s = fold_states<8>(a, M, wv, NW, count, [&](int i) { return index(row, i); });
-    if (k > 0) __syncthreads();
+  const int row = r0 + (RPW == 1 ? 0 : wv);
+  if (row >= a.R) return;  // RPW == 1: the whole workgroup
+  const float M = max_of_states(a, count, [&](int i) { return index(row, i); });
+  RowSum s = {};
+  if (M != kNegInf)
+    s = RPW == 1 ? fold_states<8>(a, M, wv, NW, count, [&](int i) { return index(row, i); })
+                 : fold_states<8>(a, M, 0, 1, count, [&](int i) { return index(row, i); });
+  if constexpr (RPW == 1) {
+    __shared__ float part[NW][kDV + 64];  // a wave's A (lane-major), then its L
+    const int lane = threadIdx.x & 63;
     reinterpret_cast<float4*>(part[wv])[2 * lane] = make_float4(s.A[0], s.A[1], s.A[2], s.A[3]);
     reinterpret_cast<float4*>(part[wv])[2 * lane + 1] = make_float4(s.A[4], s.A[5], s.A[6], s.A[7]);
     if (lane == 0) part[wv][kDV] = s.L;
     __syncthreads();
-    if (wv == 0) {
-      RowSum t = {};
+    if (wv != 0) return;
+    s = {};
 #pragma unroll
-      for (int x = 0; x < NW; ++x) {
-        const float4 v0 = reinterpret_cast<const float4*>(part[x])[2 * lane];
-        const float4 v1 = reinterpret_cast<const float4*>(part[x])[2 * lane + 1];
-        const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-        t.L += part[x][kDV];
+    for (int x = 0; x < NW; ++x) {
+      const float4 v0 = reinterpret_cast<const float4*>(part[x])[2 * lane];
+      const float4 v1 = reinterpret_cast<const float4*>(part[x])[2 * lane + 1];
+      const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+      s.L += part[x][kDV];
 #pragma unroll
-        for (int d = 0; d < 8; ++d) t.A[d] += v[d];
-      }
-      store_row(a, b, row, M, t);
+      for (int d = 0; d < 8; ++d) s.A[d] += v[d];
     }
   }
+  store_row(a, b, row, M, s);
 }
 
 // Fixed splits: the num_splits states of each row.
@@ -997,7 +987,8 @@ hipError_t make_args(mla::MlaArgs* a, const uint16_t* q, const uint16_t* kv_cach
 }
 
 hipError_t launch_splitkv(const mla::MlaArgs& a, hipStream_t stream) {
-  if (mla::wide_splitkv(a)) return mla::launch_wide_splitkv(a, stream);
+  const int rows = mla::wide_rows_splitkv(a, gqa::device_cu_count());
+  if (mla::wide_splitkv(a, rows)) return mla::launch_wide_splitkv(a, rows, stream);
   const dim3 grid((unsigned)((a.R + mla::kRowsPerGroup - 1) / mla::kRowsPerGroup), a.B,
                   a.num_splits);
   if (a.block_size % mla::kTile == 0)
@@ -1008,11 +999,13 @@ hipError_t launch_splitkv(const mla::MlaArgs& a, hipStream_t stream) {
 }
 
 // Rows of up to `pieces` states each: one row per workgroup of 16 waves where
-// rows are few and pieces many, else 4 rows per workgroup of 4 waves. One
+// rows are few and pieces many, else a wave per row, 4 rows a workgroup. One
 // request of 4096 tokens and 128 rows at 128 pieces: the fold alone took 51.7
 // us with a wave per row (32 workgroups, 16 round trips each). At 512 rows
 // (4 requests of 256 to 1024 tokens) 16 waves per row lose 10-20 % of the step
-// to 4, at 1024 rows up to a third.
+// to a wave per row, at 1024 rows up to a third; 4 waves per row lose too (512
+// rows per request, 2 requests of 9221 tokens in 32 pieces: step 49.8 us with
+// a wave per row, 57.8 with 4).
 bool merge_wide(const mla::MlaArgs& a, int64_t pieces) {
   return pieces >= 16 && (int64_t)a.B * a.R <= 256;
 }
@@ -1132,9 +1125,13 @@ extern "C" int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_
   a.pre = reinterpret_cast<uint64_t*>(ws + align16(states * (mla::kDV + 2) * sizeof(float)));
   a.nshare = n;
   const unsigned rg = (unsigned)((a.R + mla::kRowsPerGroup - 1) / mla::kRowsPerGroup);
-  if (mla::wide_balanced(a)) {
+  const int nwg = num_workgroups > 0 ? num_workgroups : gqa::device_cu_count();
+  const int rows = mla::wide_rows_balanced(a, nwg);
+  if (mla::wide_balanced(a, rows)) {
+    // (At most the n shares the workspace holds: rows <= 128.)
+    a.nshare = std::max(1, std::min(n, nwg / mla::row_groups(a.R, rows)));
     a.piece_cost = mla::kWidePieceCost;
-    if ((err = mla::launch_wide_balanced(a, stream)) != hipSuccess) return err;
+    if ((err = mla::launch_wide_balanced(a, rows, stream)) != hipSuccess) return err;
     return launch_balanced_merge(a, stream);
   }
   if (block_size % mla::kTile == 0)

@@ -13,35 +13,70 @@ namespace mla {
 // rows: 115 / 114 / 113.5 / 113 us at 0 / 2 / 4 / 8).
 constexpr int kWidePieceCost = 8;
 
-// Block sizes that are multiples of 32: a tile's rows lie in one block, so a
-// wave's copies need one scalar block id (the per-lane gather of other sizes
-// keeps to the 8-wave kernels, which have registers for it). Past 64 rows the
-// 8-wave kernels also keep
-//  - fixed splits (num_splits > 1) of at most 2048 tokens of the longest
-//    sequence: twice the waves load Q and store the states, which weighs more
-//    than the tiles there (64 requests of ~1024 tokens at 4 splits, 128 rows:
-//    51.8 against 55.5 us; of ~4096 tokens: 124.6 against 121.3);
-//  - balanced launches of at most 8 tiles in all (one request of 64 tokens:
-//    18.9 against 19.4 us; of 1024: 23.9 against 22.9).
 // (The phase-timing build stamps the 8-wave kernels, and runs them alone.)
 #ifndef MLA_PHASE_TIMING
 #define MLA_PHASE_TIMING 0
 #endif
+// Block sizes that are multiples of 32: a tile's rows lie in one block, so a
+// wave's copies need one scalar block id (the per-lane gather of other sizes
+// keeps to the 8-wave kernels, which have registers for it).
 inline bool wide_blocks(const MlaArgs& a) {
   return !MLA_PHASE_TIMING && a.block_size % kTile == 0;
 }
 inline int64_t tile_bound(const MlaArgs& a) {  // tiles of the longest sequence
   return ((int64_t)a.max_blocks * a.block_size + kTile - 1) / kTile;
 }
-inline bool wide_splitkv(const MlaArgs& a) {
-  return wide_blocks(a) &&
-         (a.R <= 64 || a.num_splits == 1 || tile_bound(a) * kTile > 2048ll * a.num_splits);
+// Row groups of `rows` query rows: 16, 32, 64 or 128, no larger than R needs.
+inline int wide_rows(int R, int rows) {
+  const int most = R <= 16 ? 16 : R <= 32 ? 32 : R <= 64 ? 64 : 128;
+  return rows < most ? rows : most;
 }
-inline bool wide_balanced(const MlaArgs& a) {
-  return wide_blocks(a) && (a.R <= 64 || a.B * tile_bound(a) > 8);
+inline int row_groups(int R, int rows) { return (R + rows - 1) / rows; }
+
+// Rows per workgroup of a balanced launch on nwg workgroups. Large row groups
+// read the cache once and are the most work per byte; small ones spread little
+// work over more CUs (every row group's workgroups read the tiles again, from
+// the L2) and have less to load and store per piece. By work, in tiles x 16
+// rows of the longest possible batch per workgroup; us at 16 / 32 / 64 / 128
+// rows (128 heads; uniform lengths up to 4 requests, varlen beyond):
+//    4  1 request of 4096 tokens      20.5   24.5   26.0   31.4
+//    8  2 of 4096                     24.6   26.2   28.1   33.3
+//   16  4 of 4096                     29.7   28.6   34.6   39.6
+//   32  2 of 16384                    43.5   37.3   37.7   42.5
+//   64  4 of 16384                    70.6   51.2   47.5   54.0
+//  128  16 of ~4096                   90.3   60.5   48.9   56.8
+//  512  16 of ~16384                 318.8  193.6  134.1  120.8
+inline int wide_rows_balanced(const MlaArgs& a, int nwg) {
+  const int64_t work = a.B * tile_bound(a) * row_groups(a.R, 16);
+  return wide_rows(a.R, work <= 12ll * nwg ? 16 : work <= 28ll * nwg ? 32 : work <= 160ll * nwg ? 64
+                                                                                            : 128);
+}
+// Fixed splits: the largest row groups that still give every CU a workgroup.
+inline int wide_rows_splitkv(const MlaArgs& a, int cus) {
+  const int64_t pieces = (int64_t)a.B * a.num_splits;
+  int rows = 128;
+  while (rows > 16 && pieces * row_groups(a.R, rows) * 2 <= cus) rows /= 2;
+  return wide_rows(a.R, rows);
 }
 
-hipError_t launch_wide_splitkv(const MlaArgs& a, hipStream_t stream);
-hipError_t launch_wide_balanced(const MlaArgs& a, hipStream_t stream);
+// Whether the wide kernels run. At 128 rows per workgroup the 8-wave kernels
+// keep
+//  - fixed splits (num_splits > 1) of at most 2048 tokens of the longest
+//    sequence: twice the waves load Q and store the states, which weighs more
+//    than the tiles there (64 requests of ~1024 tokens at 4 splits, 128 rows:
+//    51.8 against 55.5 us; of ~4096 tokens: 124.6 against 121.3);
+//  - balanced launches of at most 8 tiles in all (one request of 64 tokens:
+//    18.9 against 19.4 us; of 1024: 23.9 against 22.9), which only a caller
+//    that asks for a few workgroups brings to 128 rows.
+inline bool wide_splitkv(const MlaArgs& a, int rows) {
+  return wide_blocks(a) &&
+         (rows < 128 || a.num_splits == 1 || tile_bound(a) * kTile > 2048ll * a.num_splits);
+}
+inline bool wide_balanced(const MlaArgs& a, int rows) {
+  return wide_blocks(a) && (rows < 128 || a.B * tile_bound(a) > 8);
+}
+
+hipError_t launch_wide_splitkv(const MlaArgs& a, int rows, hipStream_t stream);
+hipError_t launch_wide_balanced(const MlaArgs& a, int rows, hipStream_t stream);
 
 }  // namespace mla

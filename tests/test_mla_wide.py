@@ -69,13 +69,29 @@ def test_second_pass_mid_share(gpu, s_q, h_q):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("S,ns", [(4096, 2), (4160, 2), (256, 1), (320, 1)])
-def test_either_side_of_the_rules(gpu, S, ns):
-    # 2048 tokens per split, 8 tiles in all: either side runs another kernel.
-    case = make_mla_case([S], 1, 128, 64, seed=S, device="cuda")
-    want = oracle(case, False)
-    check(run(case, False, ns), want, f"S{S}/ns{ns}")
-    check(run_balanced(case, False, 256), want, f"S{S}/bal")
+@pytest.mark.parametrize("S,ns,nwg", [(4096, 2, 256), (4160, 2, 256), (256, 1, 2), (320, 1, 2)])
+def test_either_side_of_the_rules(gpu, S, ns, nwg):
+    # 2048 tokens per split; 8 tiles in all on few workgroups: either side runs
+    # another kernel. (120 requests: the splits alone fill the CUs.)
+    for lens in ([S], [S] + [70] * 119):
+        case = make_mla_case(lens, 1, 128, 64, seed=S, device="cuda")
+        want = oracle(case, False)
+        check(run(case, False, ns), want, f"S{S}/ns{ns}")
+        check(run_balanced(case, False, nwg), want, f"S{S}/bal{nwg}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s_q,h_q", [(1, 30), (1, 60), (1, 128), (2, 65), (3, 128)])
+@pytest.mark.parametrize("nwg", [1, 4, 9, 30, 256])
+def test_row_groups(gpu, s_q, h_q, nwg):
+    # The same batch at every size of row group the rules give it (few
+    # workgroups: 128 rows; many: 16), full and ragged groups, causal.
+    case = make_mla_case([700, 33, 0, 5, 64, 257], s_q, h_q, 32, pool_factor=1.5, seed=h_q,
+                         device="cuda", poison=True)
+    want = oracle(case, True)
+    check(run_balanced(case, True, nwg), want, f"n{nwg}")
+    for ns in (1, 2, 12, 40):
+        check(run(case, True, ns), want, f"ns{ns}")
 
 
 @pytest.fixture(scope="module")
@@ -143,8 +159,8 @@ def test_generated_tile_loop(asm, kernel, rw, m, mfmas):
 @pytest.mark.parametrize("S_list", [[511], [512], [4096], [9000, 40], [2000, 1, 0, 700]])
 def test_merges(gpu, s_q, h_q, S_list):
     # Rows of few and of many pieces (from 16 on, up to 256 rows: 16 waves a
-    # row; else a wave a row up to 16 pieces, 4 waves beyond), rows off the four
-    # of a workgroup, and requests that are not cut at all.
+    # row; else a wave a row), rows off the four of a workgroup, and requests
+    # that are not cut at all.
     case = make_mla_case(S_list, s_q, h_q, 64, pool_factor=1.5, seed=h_q, device="cuda",
                          poison=True)
     want = oracle(case, False)
