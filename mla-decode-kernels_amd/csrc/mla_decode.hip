@@ -800,76 +800,33 @@ __global__ __launch_bounds__(64 * NW) void mla_decode_merge_kernel(const MlaArgs
 // than shares, only the first T shares take work (one tile each), so every
 // working share is non-empty.
 
-// Workgroup (w, rg): share w of row group rg. Every workgroup first plans
-// the launch itself from seq_lens (no separate plan launch): the tile counts'
-// inclusive prefix sums over chunks of the batch (one chunk per thread, a
-// scan in P buffer 1, which the first piece does not touch before its
-// second barrier) give T, the working share count n = min(nshare, T), the
-// share's tiles and its first request. Workgroup (0, 0) also writes the
-// request prefix sums pre[b] (b = 0..B), pre[B] = T and pre[B + 1] = n for
-// the merge kernel, before any workgroup can return.
+// Workgroup (w, rg): share w of row group rg. Every workgroup first plans the
+// launch itself from seq_lens (plan_share, no separate plan launch), in P
+// buffer 1, which the first piece does not touch before its second barrier.
+// Workgroup (0, 0) also writes the request prefix sums for the merge kernel,
+// before any workgroup can return.
 template <bool kBlockUniform>
 __global__ __launch_bounds__(kThreads, 1) void mla_decode_balanced_kernel(const MlaArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kLdsBytes];
   const int w = blockIdx.x, rg = blockIdx.y;
-  const int s_cap = a.max_blocks * a.block_size;
-  auto tiles_of = [&](int b) -> uint64_t {
-    const int S = min(max(a.seq_lens[b], 0), s_cap);
-    return (uint64_t)((S + kTile - 1) / kTile);
-  };
-  uint64_t* const part = reinterpret_cast<uint64_t*>(smem + kDepth * kTileBytes + kPBytes);
-  const int tid = threadIdx.x;
-  const int per = (a.B + kThreads - 1) / kThreads;
-  const int b0 = min(tid * per, a.B), b1 = min(b0 + per, a.B);
-  uint64_t sum = 0;
-  for (int b = b0; b < b1; ++b) sum += tiles_of(b);
-  part[tid] = sum;
-  __syncthreads();
-  for (int off = 1; off < kThreads; off <<= 1) {  // inclusive scan of the chunk sums
-    const uint64_t v = tid >= off ? part[tid - off] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  const uint64_t T = part[kThreads - 1];
-  const int n = (int)(T < (uint64_t)a.nshare ? T : (uint64_t)a.nshare);
-  if (w == 0 && rg == 0) {
-    uint64_t run = part[tid] - sum;
-    for (int b = b0; b < b1; ++b) {
-      a.pre[b] = run;
-      run += tiles_of(b);
-    }
-    if (tid == 0) {
-      a.pre[a.B] = T;
-      a.pre[a.B + 1] = (uint64_t)n;
-    }
-  }
-  if (w >= n) return;
-  const uint64_t t0 = share_start(T, w, n), t_end = share_start(T, w + 1, n);
-  // The share's first request: the first b whose tiles end past t0 (the
-  // chunk first, by bisection of the chunk prefix sums, then within it).
-  int lo = 0, hi = kThreads - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (part[mid] > t0) hi = mid; else lo = mid + 1;
-  }
-  uint64_t p0 = lo > 0 ? part[lo - 1] : 0;  // tiles before request b
-  int b = lo * per;
-  for (uint64_t nt = tiles_of(b); p0 + nt <= t0; nt = tiles_of(b)) {
-    p0 += nt;
-    ++b;
-  }
+  const SharePlan sp = plan_share<kThreads>(
+      a, w, reinterpret_cast<uint64_t*>(smem + kDepth * kTileBytes + kPBytes), false,
+      w == 0 && rg == 0);
+  if (sp.units <= 0) return;
+  int b = sp.b;
+  uint64_t p0 = 0;  // request b's first tile, counted from request sp.b's
+  const uint64_t t0 = (uint64_t)(sp.ts / kTile), t_end = t0 + (uint64_t)sp.units;
 #if MLA_PHASE_TIMING
   const uint64_t k_t0 = __builtin_amdgcn_s_memtime(), k_r0 = __builtin_amdgcn_s_memrealtime();
 #endif
   for (uint64_t t = t0; t < t_end; ++b) {
-    const uint64_t p1 = p0 + tiles_of(b);
+    const uint64_t p1 = p0 + tiles_of(a, b);
     if (p1 <= t) {  // a request with no tiles
       p0 = p1;
       continue;
     }
     const uint64_t t1 = p1 < t_end ? p1 : t_end;
-    const int S = min(max(a.seq_lens[b], 0), s_cap);
+    const int S = live_len(a, b);
     PieceOut po;
     po.direct = t == p0 && t1 == p1;
     po.st_base = (size_t)(2 * w + (t == t0 ? 0 : 1)) * a.R;

@@ -665,11 +665,11 @@ template <int RW, int M>
 __global__ __launch_bounds__(kWThreads, 1) void mla_wide_balanced_kernel(const MlaArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kWLds];
   const int w = blockIdx.x, rg = blockIdx.y;
-  const SharePlan sp = plan_share<kWThreads>(a, w, reinterpret_cast<uint64_t*>(smem),
+  const SharePlan sp = plan_share<kWThreads>(a, w, reinterpret_cast<uint64_t*>(smem), true,
                                              w == 0 && rg == 0);
   if (sp.units <= 0) return;
   __syncthreads();
-  wide_run<RW, M>(a, smem, rg, piece_at(a, sp.b, sp.ts, sp.units), sp.units,
+  wide_run<RW, M>(a, smem, rg, piece_of(sp.b, sp.S, sp.ts, sp.units), sp.units,
                   [&](const Piece& p, bool first) {
                     PieceOut po;
                     po.direct = p.start == 0 && p.end == p.S;

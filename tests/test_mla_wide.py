@@ -155,6 +155,20 @@ def test_generated_tile_loop(asm, kernel, rw, m, mfmas):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bs", [16, 32])  # the 8-wave kernel's plan, the others'
+@pytest.mark.parametrize("B", [1, 63, 65, 255, 257, 513, 1100])
+def test_plan_of_many_requests(gpu, B, bs):
+    # One request per planning thread and several, empty ones in between, at
+    # the ends of a wave's lanes too, and shares that start in each of them.
+    S_list = [(37 * b) % 71 if b % 5 or b % 64 in (0, 63) else 0 for b in range(B)]
+    S_list[-1] = 33
+    case = make_mla_case(S_list, 1, 4, bs, pool_factor=1.2, seed=B, device="cuda", poison=True)
+    want = oracle(case, False)
+    for nwg in (1, 40, 256, 1500):
+        check(run_balanced(case, False, nwg), want, f"bal n{nwg}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("s_q,h_q", [(1, 5), (1, 128), (2, 100), (2, 128), (3, 128)])
 @pytest.mark.parametrize("S_list", [[511], [512], [4096], [9000, 40], [2000, 1, 0, 700]])
 def test_merges(gpu, s_q, h_q, S_list):
