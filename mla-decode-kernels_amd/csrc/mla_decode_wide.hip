@@ -1,5 +1,5 @@
 // MLA absorbed-path paged decode on one wave per SIMD, for block sizes that
-// keep a 32-token tile inside one cache block (multiples of 32).
+// keep 8 aligned tokens inside one cache block (multiples of 8).
 //
 // A workgroup of 4 waves owns M x RW query rows of a request (RW rows for
 // each of M row sets) and walks the tiles of its pieces. Every tile is copied
@@ -271,12 +271,18 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
   bool c_live = true;
   uint32_t c_slot = 0;
   const int bs = a.block_size;
+  // The first token this wave copies: of its row block, or the tile's first one
+  // if the row block lies past the piece's end.
+  auto cursor_token = [&]() -> int {
+    const int t = c_ts + 8 * w;
+    return t < c.end ? t : c_ts;
+  };
   auto cursor_block = [&]() -> int {
     // The table is read-only for the launch; through the constant address
     // space the uniform block-id loads are scalar.
     return ((const __attribute__((address_space(4))) int*)(a.block_table + (size_t)c.b *
                                                                              a.max_blocks))
-        [gqa::fastdiv((uint32_t)c_ts, a.bs_div)];
+        [gqa::fastdiv((uint32_t)cursor_token(), a.bs_div)];
   };
   auto advance = [&]() {
     c_slot = c_slot + 1 < kWDepth ? c_slot + 1 : 0;
@@ -295,11 +301,12 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
   auto source = [&](int id) -> Source {
     Source s;
     s.slot = smem_lds + c_slot * kTileBytes + (uint32_t)w * kRowBlockBytes;
-    const uint32_t lb = gqa::fastdiv((uint32_t)c_ts, a.bs_div);
-    s.base = a.kv + ((size_t)id * bs + (c_ts - (int)lb * bs)) * kD;
-    // Rows past the piece's end read the tile's first row (masked later).
+    const int t = cursor_token();
+    const uint32_t lb = gqa::fastdiv((uint32_t)t, a.bs_div);
+    s.base = a.kv + ((size_t)id * bs + (t - (int)lb * bs)) * kD;
+    // Rows past the piece's end read that token's row (masked later).
     const int valid = c_live ? c.end - c_ts - 8 * w : 0;
-    s.voff = copy_row() < valid ? ro + (uint32_t)(8 * w * kD * 2) : (ro & 0x70u);
+    s.voff = copy_row() < valid ? ro : (ro & 0x70u);
     return s;
   };
   auto copy = [&](const Source& s, int i) {

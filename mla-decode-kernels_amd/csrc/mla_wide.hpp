@@ -17,11 +17,11 @@ constexpr int kWidePieceCost = 8;
 #ifndef MLA_PHASE_TIMING
 #define MLA_PHASE_TIMING 0
 #endif
-// Block sizes that are multiples of 32: a tile's rows lie in one block, so a
-// wave's copies need one scalar block id (the per-lane gather of other sizes
-// keeps to the 8-wave kernels, which have registers for it).
+// Block sizes that are multiples of 8: the 8 rows of a tile that a wave copies
+// lie in one block, so its copies need one scalar block id (the per-lane gather
+// of other sizes keeps to the 8-wave kernels, which have registers for it).
 inline bool wide_blocks(const MlaArgs& a) {
-  return !MLA_PHASE_TIMING && a.block_size % kTile == 0;
+  return !MLA_PHASE_TIMING && a.block_size % 8 == 0;
 }
 inline int64_t tile_bound(const MlaArgs& a) {  // tiles of the longest sequence
   return ((int64_t)a.max_blocks * a.block_size + kTile - 1) / kTile;

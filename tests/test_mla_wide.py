@@ -45,6 +45,24 @@ def test_rows_and_tile_edges(gpu, s_q, h_q, bs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("s_q,h_q", [(1, 3), (1, 16), (1, 32), (1, 64), (2, 64), (1, 129)])
+@pytest.mark.parametrize("bs", [4, 8, 16, 24, 40, 56])  # (4: the per-lane gather)
+def test_tiles_over_several_blocks(gpu, s_q, h_q, bs):
+    # A tile's four row blocks lie in up to four cache blocks; the last ones past
+    # a request's end have no block (their table entries are -1 or the next
+    # request's), in first, last and only tiles, and at the table's end.
+    lens = EDGES + [7, 8, 9, 15, 16, 17, 23, 24, 25, 39, 40, 41, 302, 311]
+    case = make_mla_case(lens, s_q, h_q, bs, pool_factor=1.5, seed=h_q + bs, device="cuda",
+                         poison=True)
+    for causal in {False, s_q > 1}:
+        want = oracle(case, causal)
+        for nwg in (1, 3, 40, 256):
+            check(run_balanced(case, causal, nwg), want, f"bal n{nwg}/c{causal}")
+        for ns in (1, 2, 7):
+            check(run(case, causal, ns), want, f"ns{ns}/c{causal}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("s_q,h_q", [(1, 16), (1, 32), (1, 64), (1, 128)])
 def test_second_pass_mid_share(gpu, s_q, h_q):
     # Keys that beat everything else by more than 128 log2 units (fp32 overflows
@@ -155,7 +173,7 @@ def test_generated_tile_loop(asm, kernel, rw, m, mfmas):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("bs", [16, 32])  # the 8-wave kernel's plan, the others'
+@pytest.mark.parametrize("bs", [16, 32])
 @pytest.mark.parametrize("B", [1, 63, 65, 255, 257, 513, 1100])
 def test_plan_of_many_requests(gpu, B, bs):
     # One request per planning thread and several, empty ones in between, at
@@ -166,6 +184,13 @@ def test_plan_of_many_requests(gpu, B, bs):
     want = oracle(case, False)
     for nwg in (1, 40, 256, 1500):
         check(run_balanced(case, False, nwg), want, f"bal n{nwg}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [65, 257, 1100])
+def test_plan_of_many_requests_gathered(gpu, B):
+    # The 8-wave kernel's plan (block sizes off 8).
+    test_plan_of_many_requests(gpu, B, 4)
 
 
 @pytest.mark.gpu
