@@ -7,10 +7,12 @@
 namespace mla {
 
 // What a piece weighs besides its tiles in the balanced plan, in tiles: Q, the
-// first tile's scores, the last tile's PV and the stores take 10-14 us per
-// piece of 128 rows against ~1.8 us per tile (mla_4k: 187 / 185 / 182 us at 2 /
-// 4 / 8). Fewer rows: 3-4 us against 1.4 (128 requests of ~4096 tokens, 16
-// rows: 115 / 114 / 113.5 / 113 us at 0 / 2 / 4 / 8).
+// first tile's scores, the last tile's PV and the stores, 12-14 us per piece of
+// 128 rows against 2.6 us per tile and 7 against 1.3 with 16 rows (fits over
+// the workgroups of 128 requests of ~4096 tokens). Step at 2 / 4 / 6 / 8 / 10:
+//    that batch, 128 heads       184.8 / 180.7 / 175.0 / 173.1 / 176.0 us
+//    that batch, 16 heads        109.0 / 108.5 / 109.1 / 109.7 / 110.2 us
+//    64 requests of ~2000        76.2 / 73.1 / 69.1 / 68.7 / 68.8 us
 constexpr int kWidePieceCost = 8;
 
 // (The phase-timing build stamps the 8-wave kernels, and runs them alone.)
@@ -20,6 +22,9 @@ constexpr int kWidePieceCost = 8;
 // Block sizes that are multiples of 8: the 8 rows of a tile that a wave copies
 // lie in one block, so its copies need one scalar block id (the per-lane gather
 // of other sizes keeps to the 8-wave kernels, which have registers for it).
+// 16-token blocks, the gather -> here: one request of 4096 tokens, 128 heads,
+// 75.9 -> 20.0 us (its smaller row groups with it); 128 requests of ~4096
+// tokens 195.4 -> 179.1 (128 heads) and 144.0 -> 112.0 (16 heads).
 inline bool wide_blocks(const MlaArgs& a) {
   return !MLA_PHASE_TIMING && a.block_size % 8 == 0;
 }
