@@ -322,10 +322,12 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
   acc_t o[kBlocks];
   acc_t c4[Sh::kChains];  // QK^T accumulators
   float e[Sh::kEl];       // the exponents of the tile whose probabilities come next
-  float lsum = 0.f;
-  float mref = kNegInf;  // the row's reference (log2 units); -inf until its first live tile
-  float nbase = 0.f;     // -mref (0 before the first live tile)
-  float mrel = kNegInf;  // largest exponent of this lane's tokens, relative to mref
+  float lsum = 0.f;      // the row's probabilities, before their rounding to bf16
+  float lpv = 0.f;       // and as PV multiplies them
+  float nbase = 0.f;     // less the row's reference (log2 units); 0 until its first live tile
+  // Largest exponent of this lane's tokens, relative to the reference, and at
+  // least 0 (the tile that set it); -inf until the row's first live tile.
+  float mrel = kNegInf;
   int d = 0;             // the lane's score i of the tile is live iff tok_off(i) < d
 
   uint32_t g0 = 0;  // ring slot of the piece's first tile
@@ -360,11 +362,20 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
                    o[nb]);
   };
   auto settle = [&](int i) { e[i] = Sh::exponent(c4, i, a.scale_log2e, nbase); };
-  // PV takes the probabilities rounded to bf16; l sums them before the rounding
-  // (lse against float64: 5e-7 rms; from the rounded ones 2e-5 to 6e-5).
+  // PV takes the probabilities rounded to bf16. Its normaliser sums the rounded
+  // ones too, so that an output is a weighted mean of its value rows (with the
+  // unrounded sum a constant value column of 16 tokens came back up to 1e-3
+  // off); lse takes the sum before the rounding (against float64 5e-7 rms; from
+  // the rounded ones 2e-5 to 6e-5).
   auto pack_probs = [&](int k, float x, float y) {
     pw[k] = pack_bf16(x, y);
     lsum += x + y;
+  };
+  auto sum_packed = [&]() {
+    asm volatile("" : "+v"(lpv));  // (kept where it is called)
+#pragma unroll
+    for (int k = 0; k < Sh::kEl / 2; ++k) lpv = gqa::dot2_bf16(pw[k], 0x3F803F80u, lpv);
+    asm volatile("" : "+v"(lpv));
   };
   auto max_of = [&]() {
     float m = fmaxf(e[0], e[1]);
@@ -375,13 +386,13 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
   // A tile with masked tokens, or a row's first live tile (its maximum becomes
   // the row's reference): rare, behind a uniform branch.
   auto check_tile = [&](float mx) {
-    if (__builtin_amdgcn_ballot_w64(d <= Sh::kMaxTok || mref == kNegInf) != 0) {
+    if (__builtin_amdgcn_ballot_w64(d <= Sh::kMaxTok || mrel == kNegInf) != 0) {
 #pragma unroll
       for (int i = 0; i < Sh::kEl; ++i) e[i] = Sh::tok_off(i) < d ? e[i] : kNegInf;
       const float m = Sh::row_max(max_of());
-      const float delta = mref == kNegInf && m != kNegInf ? m : 0.f;
-      mref = mref == kNegInf ? m : mref;
-      nbase = mref == kNegInf ? 0.f : -mref;
+      const float delta = mrel == kNegInf && m != kNegInf ? m : 0.f;
+      mrel = m != kNegInf ? fmaxf(mrel, 0.f) : mrel;
+      nbase -= delta;
 #pragma unroll
       for (int i = 0; i < Sh::kEl; ++i) e[i] -= delta;
       mx = max_of();
@@ -411,9 +422,9 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
       const int end = a.causal ? p.S - (a.s_q - 1 - query_row(l) / a.h_q) : p.S;
       d = min(p.end, end) - 4 * (l / RW) - p.start;
     }
-    lsum = 0.f;
+    lsum = lpv = 0.f;
     if (!again) {
-      mref = mrel = kNegInf;
+      mrel = kNegInf;
       nbase = 0.f;
     }
 #pragma unroll
@@ -482,6 +493,13 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
           set_ka(s + 2);
 #pragma unroll
           for (int k = 0; k < kWKRing - 1; ++k) read_k(k);
+          // Summed here because the MFMAs wait for these reads anyway (128
+          // heads, 128 requests of ~4096 tokens / the same with s_q = 2 / of
+          // ~16384 with s_q = 2: 171 / 300 / 1046 us with the 8 instructions
+          // between the QK^T MFMAs, 169 / 292 / 992 here, 169 / 290 / 994
+          // without them).
+          __builtin_amdgcn_sched_barrier(0);
+          sum_packed();
         }
         __builtin_amdgcn_sched_barrier(0);
         pv_mfma(i);
@@ -524,6 +542,8 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
         pack_probs(k, exp2_fast(e[2 * k]), exp2_fast(e[2 * k + 1]));
 #pragma unroll
       for (int i = 0; i < kWVRing - 1; ++i) read_v(T, i);
+      __builtin_amdgcn_sched_barrier(0);
+      sum_packed();
 #pragma unroll
       for (int i = 0; i < kPv; ++i) {
         if (i + kWVRing - 1 < kPv) read_v(T, i + kWVRing - 1);
@@ -550,8 +570,7 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
     if (__builtin_amdgcn_readfirstlane(v.x | v.y | v.z | v.w) != 0) {
       // Some row's later tile beat its reference by more than kWSlack: the
       // piece runs again, the copies start over at its first tile.
-      mref += fmaxf(Sh::row_max(mrel), 0.f);
-      nbase = mref == kNegInf ? 0.f : -mref;
+      nbase -= fmaxf(Sh::row_max(mrel), 0.f);
       again = true;
       publish_barrier<0>();
       c = p;
@@ -572,19 +591,20 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
     const PieceOut po = out_of(p, first);
     const bool direct = uniform((int)po.direct) != 0;
     if (row0 < a.R) {
-      const float L = Sh::row_sum(lsum);
-      const float inv = L > 0.f ? 1.f / L : 0.f;
+      const float L = Sh::row_sum(lsum), Lpv = Sh::row_sum(lpv);
+      // out = o / Lpv; a state's rows, normalised by its L later on, o L / Lpv.
+      const float factor = L > 0.f ? (direct ? 1.f : L) / Lpv : direct ? 0.f : 1.f;
       const int l = fresh_lane();
       const int row = row0 + l % RW;
       if (row < a.R && l < RW && part == 0) {
         if (!direct) {
           const size_t sx = po.st_base + (size_t)row * po.st_stride;
-          a.ws_m[sx] = L > 0.f ? mref * kLn2 : kNegInf;  // natural-log units
+          a.ws_m[sx] = L > 0.f ? -nbase * kLn2 : kNegInf;  // natural-log units
           a.ws_l[sx] = L;
         } else if (a.lse) {
           const int qi = row / a.h_q, hq = row - qi * a.h_q;
           a.lse[((size_t)p.b * a.h_q + hq) * a.s_q + qi] =
-              L > 0.f ? mref * kLn2 + logf(L) : kNegInf;
+              L > 0.f ? logf(L) - nbase * kLn2 : kNegInf;
         }
       }
       const uint32_t buf =
@@ -592,12 +612,12 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
       const uint32_t dst = buf + (uint32_t)(l % RW) * 256;
       // This lane's rows 4 i + l / 16: what it reads back and stores. (Past the
       // last row: the last row's values once more.)
-      float iv[RW / 4];
+      float fr[RW / 4];
       uint32_t off[RW / 4];
 #pragma unroll
       for (int i = 0; i < RW / 4; ++i) {
         const int r = 4 * i + (l >> 4);
-        iv[i] = __shfl(inv, r, 64);
+        fr[i] = __shfl(factor, r, 64);
         off[i] = (uint32_t)min(r, a.R - 1 - row0);
       }
       const int dim0 = part * (kDV / kParts) + 4 * (l & 15);
@@ -627,12 +647,14 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
 #pragma unroll
           for (int i = 0; i < RW / 4; ++i)
             *reinterpret_cast<uint2*>(out0 + off[i] * kDV + 64 * k) =
-                make_uint2(pack_bf16(__uint_as_float(v[i].x) * iv[i], __uint_as_float(v[i].y) * iv[i]),
-                           pack_bf16(__uint_as_float(v[i].z) * iv[i], __uint_as_float(v[i].w) * iv[i]));
+                make_uint2(pack_bf16(__uint_as_float(v[i].x) * fr[i], __uint_as_float(v[i].y) * fr[i]),
+                           pack_bf16(__uint_as_float(v[i].z) * fr[i], __uint_as_float(v[i].w) * fr[i]));
         } else {
 #pragma unroll
           for (int i = 0; i < RW / 4; ++i)
-            *reinterpret_cast<u32x4_t*>(acc0 + off[i] * pitch + 64 * k) = v[i];
+            *reinterpret_cast<float4*>(acc0 + off[i] * pitch + 64 * k) =
+                make_float4(__uint_as_float(v[i].x) * fr[i], __uint_as_float(v[i].y) * fr[i],
+                            __uint_as_float(v[i].z) * fr[i], __uint_as_float(v[i].w) * fr[i]);
         }
       }
     }

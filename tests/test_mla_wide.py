@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 import torch
 
+import capi
 from cases import make_mla_case
 from test_mla import SCALE, check, oracle, run, run_balanced
 from test_mla_codegen import HIPCC, ROOT, kernel_body, tile_loops
@@ -110,6 +111,46 @@ def test_row_groups(gpu, s_q, h_q, nwg):
     check(run_balanced(case, True, nwg), want, f"n{nwg}")
     for ns in (1, 2, 12, 40):
         check(run(case, True, ns), want, f"ns{ns}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h_q", [16, 32, 64, 128])
+@pytest.mark.parametrize("S,ns,bs", [(16, 1, 64), (70, 2, 64), (200, 3, 64), (70, 2, 12)])
+def test_constant_value_column(gpu, h_q, S, ns, bs):
+    # A value column that is c in every token is c in the output and in the
+    # normalised fp32 states, whatever the weights: both sums of a state add the
+    # same weights, c times a bf16 weight is exact in fp32, and a sum of N
+    # positive terms is within N 2^-24 of its exact value however it is ordered.
+    # (Weights summed before their rounding to bf16: 3e-5 off.) The table is
+    # wide enough for fixed splits to take every kernel (12-token blocks: the
+    # 8-wave ones).
+    q, kv, bt, sl = make_mla_case([S] * 3, 1, h_q, bs, pool_factor=1, seed=S, device="cuda",
+                                  poison=True)
+    bt = torch.cat([bt, torch.full((3, 8192 // bs), -1, dtype=torch.int32, device="cuda")], 1)
+    case = (q, kv, bt.contiguous(), sl)
+    cols = {3: 10.0, 200: 1.0, 511: -0.7109375}  # (bf16 values)
+    for d, c in cols.items():
+        kv[..., d] = torch.where(kv[..., d].isnan(), kv[..., d], c)
+    out = torch.empty(3, 1, h_q, 512, dtype=torch.bfloat16, device="cuda")
+    lse = torch.empty(3, h_q, 1, dtype=torch.float32, device="cuda")
+    wsb = max(capi.mla_workspace_bytes(3, 1, h_q, ns), 16)
+    ws = torch.zeros(wsb // 4, dtype=torch.float32, device="cuda")
+    assert capi.mla_splitkv_launch(
+        q.data_ptr(), kv.data_ptr(), case[2].data_ptr(), sl.data_ptr(), out.data_ptr(),
+        lse.data_ptr(), 3, 1, h_q, bs, case[2].shape[1], SCALE, 0, ns, ws.data_ptr(), wsb,
+        torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    per_split = -(-(-(-S // ns)) // 32) * 32
+    if ns > 1:
+        n = 3 * h_q * ns
+        acc, l = ws[:n * 512].view(n, 512).double(), ws[n * 513:n * 514].double()
+        assert (l > 0).all()
+        for d, c in cols.items():
+            err = float((acc[:, d] / l / c - 1).abs().max())
+            assert err <= (2 * per_split + 4) * 2.0 ** -24, f"state column {d}: {err:.2e} off"
+    for got in (run_balanced(case, False, 256)[0], out if ns == 1 else run(case, False, ns)[0]):
+        for d, c in cols.items():
+            assert (got[..., d].float() == c).all()
 
 
 @pytest.fixture(scope="module")
