@@ -51,10 +51,23 @@ inline int row_groups(int R, int rows) { return (R + rows - 1) / rows; }
 //   64  4 of 16384                    70.6   51.2   47.5   54.0
 //  128  16 of ~4096                   90.3   60.5   48.9   56.8
 //  512  16 of ~16384                 318.8  193.6  134.1  120.8
+// Short requests are not that work but pieces: as long as larger row groups
+// leave fewer requests than shares, requests of up to two tiles take them (the
+// balanced launch at the rows by work -> here, and the 8-wave kernels: 200
+// requests of 16 tokens, 64 heads, 25.2 -> 15.3, 18.8 us; 256 of 64, 128 heads,
+// 38.7 -> 28.9, 33.0). Longer ones cost more in one large row group than in two
+// rounds of smaller ones, unless every round of large ones is full: 256 of 200
+// (500), 128 heads, 45.4 -> 39.8, 43.3 (66.9 -> 63.0, 61.1) us, but 300 of 200
+// 60.4 -> 65.4. (256 of ~200, ragged, pay for it: 50.2 -> 54.2, 90.6.)
 inline int wide_rows_balanced(const MlaArgs& a, int nwg) {
-  const int64_t work = a.B * tile_bound(a) * row_groups(a.R, 16);
-  return wide_rows(a.R, work <= 12ll * nwg ? 16 : work <= 28ll * nwg ? 32 : work <= 160ll * nwg ? 64
-                                                                                            : 128);
+  const int64_t tiles = tile_bound(a), work = a.B * tiles * row_groups(a.R, 16);
+  int rows = wide_rows(a.R, work <= 12ll * nwg ? 16 : work <= 28ll * nwg ? 32
+                                                  : work <= 160ll * nwg ? 64 : 128);
+  const int most = wide_rows(a.R, 128);
+  if (tiles <= 2)
+    while (rows < most && (int64_t)a.B * row_groups(a.R, rows) > nwg) rows *= 2;
+  if (tiles >= 8 && (int64_t)a.B * row_groups(a.R, most) % nwg == 0) rows = most;
+  return rows;
 }
 // Fixed splits: the largest row groups that still give every CU a workgroup.
 inline int wide_rows_splitkv(const MlaArgs& a, int cus) {

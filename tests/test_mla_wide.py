@@ -234,6 +234,34 @@ def test_plan_of_many_requests_gathered(gpu, B):
     test_plan_of_many_requests(gpu, B, 4)
 
 
+def launched_plan(case, nwg):
+    """(the requests' first units and their end [B + 1], shares per row group) of
+    a balanced launch, as its split kernel left them behind the states."""
+    q, kv, bt, sl = case
+    B, s_q, h_q, _ = q.shape
+    out = torch.empty(B, s_q, h_q, 512, dtype=torch.bfloat16, device="cuda")
+    wsb = capi.mla_balanced_workspace_bytes(B, s_q, h_q, nwg)
+    ws = torch.zeros(wsb, dtype=torch.uint8, device="cuda")
+    assert capi.mla_balanced_launch(
+        q.data_ptr(), kv.data_ptr(), bt.data_ptr(), sl.data_ptr(), out.data_ptr(), None, B, s_q,
+        h_q, kv.shape[1], bt.shape[1], SCALE, 0, nwg, ws.data_ptr(), wsb,
+        torch.cuda.current_stream().cuda_stream) == 0
+    pre = ws[wsb - 8 * (B + 2):].view(torch.int64).cpu()
+    return pre[:-1].tolist(), int(pre[-1]) & 0xFFFFFFFF
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,h_q", [(200, 16, 64), (256, 16, 16), (256, 33, 128), (256, 64, 64),
+                                     (120, 50, 128), (256, 300, 128)])
+def test_a_share_for_every_short_request(gpu, B, S, h_q):
+    # Requests that fit the workgroups one each are not put together (a share
+    # pays for its pieces one after the other).
+    case = make_mla_case([S] * B, 1, h_q, 64, pool_factor=1, seed=S, device="cuda", poison=True)
+    want = oracle(case, False)
+    check(run_balanced(case, False, 256), want, f"B{B}/S{S}/h{h_q}")
+    assert launched_plan(case, 256)[1] >= B
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("s_q,h_q", [(1, 5), (1, 128), (2, 100), (2, 128), (3, 128)])
 @pytest.mark.parametrize("S_list", [[511], [512], [4096], [9000, 40], [2000, 1, 0, 700]])
