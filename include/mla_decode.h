@@ -90,7 +90,8 @@ GQA_DECODE_API int mla_decode_combine_launch(void* workspace, size_t workspace_b
  * rounding), with the batch's work cut into equal shares whatever the lengths,
  * as FlashMLA's tile scheduler does. The work is every request's 32-token
  * tiles in request order (ceil(S_b / 32) of them), each request's behind a
- * fixed weight of a few tiles for what a request costs besides them; each row
+ * fixed weight of a few tiles for what a request costs besides them (but none in
+ * a batch of equal requests that the shares divide evenly); each row
  * group (up to 128 query rows) gets at most n = num_workgroups /
  * ceil(s_q h_q / 128) shares (num_workgroups <= 0: the device's CU count) of
  * equal weight. Two launches on `stream`: the split kernel, each of whose

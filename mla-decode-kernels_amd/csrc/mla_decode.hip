@@ -856,14 +856,15 @@ __global__ __launch_bounds__(64 * NW) void mla_decode_balanced_merge_kernel(cons
   const __attribute__((address_space(4))) uint64_t* pre =
       (const __attribute__((address_space(4))) uint64_t*)a.pre;
   const uint64_t p0 = pre[b], p1 = pre[b + 1], U = pre[a.B];
-  const int n = (int)pre[a.B + 1];
+  const uint64_t shares = pre[a.B + 1];
+  const int n = (int)(uint32_t)shares;
   if (p1 == p0) {
     const int row = r0 + (int)(threadIdx.x >> 6);
     if (threadIdx.x < 64 * RPW && row < a.R) store_row(a, b, row, kNegInf, RowSum{});
     return;
   }
   // Shares holding the request's first and last tile.
-  const int w_lo = share_of(U, p0 + (uint64_t)a.piece_cost, n);
+  const int w_lo = share_of(U, p0 + (shares >> 32), n);
   const int w_hi = share_of(U, p1 - 1, n);
   if (w_lo == w_hi) return;
   // Pieces: share w_lo's last slot (its first if no earlier request has tiles

@@ -7,12 +7,22 @@
 namespace mla {
 
 // What a piece weighs besides its tiles in the balanced plan, in tiles: Q, the
-// first tile's scores, the last tile's PV and the stores, 12-14 us per piece of
-// 128 rows against 2.6 us per tile and 7 against 1.3 with 16 rows (fits over
-// the workgroups of 128 requests of ~4096 tokens). Step at 2 / 4 / 6 / 8 / 10:
-//    that batch, 128 heads       184.8 / 180.7 / 175.0 / 173.1 / 176.0 us
-//    that batch, 16 heads        109.0 / 108.5 / 109.1 / 109.7 / 110.2 us
-//    64 requests of ~2000        76.2 / 73.1 / 69.1 / 68.7 / 68.8 us
+// first tile's scores, the last tile's PV and the stores. Fits over the
+// workgroups' ends say 5 to 6 (128 requests of ~4096 tokens: 12.5 us per piece
+// and 2.6 per tile at 128 rows, 7.5 and 1.3 at 16; 32 of ~16384, 64 rows: 8.1
+// and 1.36); at 8 the shares of one piece end last (171 us, of two 165, of three
+// 159). It is 8 because most steps are fastest there. Step (us) at
+//                                   2      4      5      6      8      10
+//  128 of ~4096, 128 heads        184.8  180.7  178.6  175.0  173.1  176.0
+//    the same, s_q = 2            305.3  304.8  302.2  300.1  300.9  301.3
+//    the same, 16 heads           109.0  108.5  109.0  109.1  109.7  110.2
+//  128 of ~8192, 128 heads        323.0  319.5  319.7  319.3  315.8  317.4
+//  64 of ~2000, 128 heads          76.2   73.1   70.6   69.1   68.7   68.8
+//  128 of ~1000, 128 heads         82.3   77.9   75.8   73.9   73.5   73.5
+//  32 of ~16384, 64 heads         117.3  114.2  114.3  114.6  113.9  113.8
+//  16 of ~4096, 128 heads          45.3   43.0   42.5   42.8   43.5   43.7
+//  7 of ~3000, 128 heads           33.7   33.6   34.0   33.9   34.2   34.1
+// (Even batches, best without: kEvenTiles.)
 constexpr int kWidePieceCost = 8;
 
 // (The phase-timing build stamps the 8-wave kernels, and runs them alone.)

@@ -263,6 +263,28 @@ def test_a_share_for_every_short_request(gpu, B, S, h_q):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("h_q", [16, 128])
+@pytest.mark.parametrize("tiles,nwg,even", [
+    ([64, 64], 4, True), ([64] * 3, 3, True), ([65] * 3, 6, True), ([100], 3, True),
+    ([64] * 4, 12, True), ([64, 64], 5, False), ([64, 65], 4, False), ([65, 64], 4, False),
+    # Not even, for all that the sum, the first and the last one say.
+    ([64, 63, 65, 64], 8, False), ([64, 0, 136, 64], 8, False)])
+def test_even_batches(gpu, tiles, nwg, even, h_q):
+    # Requests of as many tiles each (whatever their last tiles hold) that the
+    # shares divide evenly are cut without the weight of a piece, all others
+    # with it.
+    S_list = [max(0, 32 * t - (7 * i) % 32) for i, t in enumerate(tiles)]
+    case = make_mla_case(S_list, 1, h_q, 64, pool_factor=1.5, seed=nwg, device="cuda", poison=True)
+    check(run_balanced(case, False, nwg), oracle(case, False), f"{tiles}/n{nwg}/h{h_q}")
+    pre, n = launched_plan(case, nwg)
+    weight = 0 if even else 8  # kWidePieceCost
+    want = [0]
+    for t in tiles:
+        want.append(want[-1] + (t + weight if t else 0))
+    assert pre == want and n == nwg
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("s_q,h_q", [(1, 5), (1, 128), (2, 100), (2, 128), (3, 128)])
 @pytest.mark.parametrize("S_list", [[511], [512], [4096], [9000, 40], [2000, 1, 0, 700]])
 def test_merges(gpu, s_q, h_q, S_list):
