@@ -99,7 +99,9 @@ GQA_DECODE_API int mla_decode_combine_launch(void* workspace, size_t workspace_b
  * share and first request: no host synchronisation, graph-capturable; requests
  * that fall inside one share are written to out and lse directly, the pieces
  * of the others to workspace states), and a merge of the cut requests in share
- * order (bitwise reproducible for a given num_workgroups).
+ * order. Bitwise reproducible for given lengths, num_workgroups and table width
+ * (max_blocks * block_size bounds the lengths and with them decides on the row
+ * groups, so a wider table for the same requests can cut them elsewhere).
  * workspace: mla_decode_balanced_workspace_bytes(B, s_q, h_q, num_workgroups)
  * bytes, 16-byte aligned, uninitialised is fine. */
 GQA_DECODE_API int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_cache,
@@ -114,6 +116,18 @@ GQA_DECODE_API int mla_decode_balanced_launch(const uint16_t* q, const uint16_t*
  * prefix sums of the requests' weights (B + 2 uint64). */
 GQA_DECODE_API size_t mla_decode_balanced_workspace_bytes(int B, int s_q, int h_q,
                                                           int num_workgroups);
+
+/* The balanced launch's cuts as counts, FlashMLA's num_splits: num_splits
+ * [B + 1] is 0 and then, request by request, the running count of the partial
+ * results (pieces) that mla_decode_balanced_launch makes of the requests with
+ * this B, s_q, h_q, block_size, max_blocks and num_workgroups; max_blocks 0
+ * stands for a table as wide as the longest request. seq_lens and num_splits are
+ * device memory (one launch on `stream`) or, with on_host, host memory (done on
+ * return). Returns 0 or a hipError_t code. */
+GQA_DECODE_API int mla_decode_balanced_num_splits(const int* seq_lens, int* num_splits, int B,
+                                                  int s_q, int h_q, int block_size,
+                                                  int max_blocks, int num_workgroups, int on_host,
+                                                  hipStream_t stream);
 
 /* Workspace bytes for mla_decode_launch: B * s_q * h_q * num_splits * (512 + 2)
  * * 4 for num_splits > 1, 0 for num_splits == 1 or invalid arguments. */

@@ -875,6 +875,140 @@ __global__ __launch_bounds__(64 * NW) void mla_decode_balanced_merge_kernel(cons
   });
 }
 
+// ---------------------------------------------------------------------------
+// The plan's cuts as counts (FlashMLA's num_splits): num_splits[b + 1] adds the
+// pieces of request b of the balanced launch. One workgroup: the work is a few
+// loads and divisions per request, and what counts is one launch per decode step
+// (as tensor operations 140 to 490 us of host time).
+
+// The launch's row groups by the tiles of the longest sequence.
+struct CutRules {
+  static constexpr int kMost = 8;  // (balanced_rows changes at six places at most)
+  struct Rule {
+    int64_t until;  // up to this many tiles
+    int nshare, weight;
+  };
+  Rule rule[kMost + 1];
+  int count;  // the last rule's index
+  __host__ __device__ Rule of(int64_t tiles) const {
+    int i = 0;
+    while (i < count && tiles > rule[i].until) ++i;
+    return rule[i];
+  }
+};
+constexpr int64_t kMaxTiles = int64_t(1) << 26;
+
+__host__ __device__ inline int64_t tiles_of_tokens(int64_t tokens) {
+  return (tokens + kTile - 1) / kTile;
+}
+__host__ __device__ inline int64_t clamped(int len, int64_t cap) {
+  return len < 0 ? 0 : len > cap ? cap : len;
+}
+// What decides on a plan's cuts: tiles in all, tokens of the longest and the
+// shortest request, and requests with tiles.
+struct BatchSums {
+  int64_t tiles, longest, shortest, live;
+  __host__ __device__ void add(const BatchSums& o) {
+    tiles += o.tiles;
+    longest = longest > o.longest ? longest : o.longest;
+    shortest = shortest < o.shortest ? shortest : o.shortest;
+    live += o.live;
+  }
+};
+__host__ __device__ inline BatchSums sums_of(int64_t tokens) {
+  return {tiles_of_tokens(tokens), tokens, tokens, tokens > 0 ? 1 : 0};
+}
+constexpr BatchSums kNoSums{0, 0, INT64_MAX, 0};
+// The line of U units cut into n shares, a request's tiles behind `weight`
+// units (plan_share's rules).
+struct Cuts {
+  uint64_t U;
+  int n, weight;
+  // Pieces of a request whose units end at `end`.
+  __host__ __device__ int pieces(uint64_t end, uint64_t tiles) const {
+    if (tiles == 0) return 0;
+    const uint64_t first = end - tiles;
+    return (int)((end * (uint64_t)n - 1) / U - ((first + 1) * (uint64_t)n - 1) / U) + 1;
+  }
+};
+__host__ __device__ inline Cuts cuts_of(const BatchSums& s, int B, int block_size,
+                                        const CutRules& rules) {
+  // (A table as wide as the longest request, in whole blocks.)
+  const CutRules::Rule r =
+      rules.of(tiles_of_tokens((s.longest + block_size - 1) / block_size * block_size));
+  Cuts c{(uint64_t)(s.tiles + s.live * r.weight), 0, r.weight};
+  c.n = r.weight ? share_count(c.U, B, r.nshare)
+                 : (int)(c.U < (uint64_t)r.nshare ? c.U : (uint64_t)r.nshare);
+  if (r.weight && s.shortest > 0 && tiles_of_tokens(s.shortest) == tiles_of_tokens(s.longest) &&
+      s.tiles >= (int64_t)kEvenTiles * c.n && c.n % B == 0) {
+    c.weight = 0;
+    c.U = (uint64_t)s.tiles;
+  }
+  return c;
+}
+
+inline void host_num_splits(const int* lens, int* out, int B, int block_size, int64_t cap,
+                            const CutRules& rules) {
+  BatchSums s = kNoSums;
+  for (int b = 0; b < B; ++b) s.add(sums_of(clamped(lens[b], cap)));
+  const Cuts c = cuts_of(s, B, block_size, rules);
+  uint64_t end = 0;
+  out[0] = 0;
+  for (int b = 0; b < B; ++b) {
+    const int64_t t = tiles_of_tokens(clamped(lens[b], cap));
+    end += t > 0 ? (uint64_t)(t + c.weight) : 0;
+    out[b + 1] = out[b] + c.pieces(end, (uint64_t)t);
+  }
+}
+
+constexpr int kNumSplitsThreads = 256;
+__global__ __launch_bounds__(kNumSplitsThreads) void mla_num_splits_kernel(
+    const int* lens, int* out, int B, int block_size, int64_t cap, const CutRules rules) {
+  constexpr int NW = kNumSplitsThreads / 64;
+  __shared__ BatchSums wave_sums[NW];
+  __shared__ uint64_t scans[2][NW];
+  const int tid = threadIdx.x, wv = tid >> 6;
+  const int per = (B + kNumSplitsThreads - 1) / kNumSplitsThreads;
+  const int b0 = min(tid * per, B), b1 = min(b0 + per, B);
+  BatchSums s = kNoSums;
+  for (int b = b0; b < b1; ++b) s.add(sums_of(clamped(lens[b], cap)));
+  const uint64_t own_tiles = (uint64_t)s.tiles, own_live = (uint64_t)s.live;
+  for (int d = 32; d > 0; d >>= 1) {
+    const BatchSums o{__shfl_xor(s.tiles, d, 64), __shfl_xor(s.longest, d, 64),
+                      __shfl_xor(s.shortest, d, 64), __shfl_xor(s.live, d, 64)};
+    s.add(o);
+  }
+  if ((tid & 63) == 0) wave_sums[wv] = s;
+  __syncthreads();
+  s = wave_sums[0];
+  for (int k = 1; k < NW; ++k) s.add(wave_sums[k]);
+  const Cuts c = cuts_of(s, B, block_size, rules);
+  // Sum over the threads before this one.
+  auto before = [&](uint64_t sum, int which) -> uint64_t {
+    uint64_t x = wave_scan(sum);
+    if ((tid & 63) == 63) scans[which][wv] = x;
+    __syncthreads();
+    for (int k = 0; k < wv; ++k) x += scans[which][k];
+    return x - sum;
+  };
+  const uint64_t first = before(own_tiles + own_live * (uint64_t)c.weight, 0);
+  uint64_t end = first, pieces = 0;
+  for (int b = b0; b < b1; ++b) {
+    const int64_t t = tiles_of_tokens(clamped(lens[b], cap));
+    end += t > 0 ? (uint64_t)(t + c.weight) : 0;
+    pieces += (uint64_t)c.pieces(end, (uint64_t)t);
+  }
+  int at = (int)before(pieces, 1);
+  if (tid == 0) out[0] = 0;
+  end = first;
+  for (int b = b0; b < b1; ++b) {
+    const int64_t t = tiles_of_tokens(clamped(lens[b], cap));
+    end += t > 0 ? (uint64_t)(t + c.weight) : 0;
+    at += c.pieces(end, (uint64_t)t);
+    out[b + 1] = at;
+  }
+}
+
 }  // namespace mla
 
 extern "C" size_t mla_decode_workspace_bytes(int B, int s_q, int h_q, int num_splits) {
@@ -1049,6 +1183,11 @@ int balanced_shares(int s_q, int h_q, int num_workgroups) {
   return (int)std::min<int64_t>(kMaxShares, std::max<int64_t>(1, num_workgroups / rg));
 }
 
+// Those of the wide kernels (at most the n that the workspace holds).
+int wide_shares(int n, int R, int rows, int nwg) {
+  return std::max(1, std::min(n, nwg / mla::row_groups(R, rows)));
+}
+
 size_t align16(size_t x) { return (x + 15) & ~size_t(15); }
 
 }  // namespace
@@ -1059,6 +1198,44 @@ extern "C" size_t mla_decode_balanced_workspace_bytes(int B, int s_q, int h_q, i
   if (n <= 0) return 0;
   const size_t states = (size_t)2 * n * s_q * h_q;
   return align16(states * (mla::kDV + 2) * sizeof(float)) + (size_t)(B + 2) * 8;
+}
+
+extern "C" int mla_decode_balanced_num_splits(const int* seq_lens, int* num_splits, int B, int s_q,
+                                              int h_q, int block_size, int max_blocks,
+                                              int num_workgroups, int on_host,
+                                              hipStream_t stream) {
+  if (B < 0 || s_q < 1 || h_q < 1 || block_size < 1 || max_blocks < 0 || !num_splits ||
+      (B > 0 && !seq_lens))
+    return hipErrorInvalidValue;
+  if ((int64_t)s_q * h_q > (int64_t(1) << 20) ||
+      (int64_t)block_size * max_blocks >= (int64_t(1) << 31))
+    return hipErrorInvalidValue;
+  const int n = balanced_shares(s_q, h_q, num_workgroups);
+  if (n <= 0) return hipErrorInvalidValue;
+  const int nwg = num_workgroups > 0 ? num_workgroups : gqa::device_cu_count();
+  const int R = s_q * h_q;
+  mla::CutRules rules;
+  int64_t tiles = max_blocks > 0 ? mla::tiles_of_tokens((int64_t)max_blocks * block_size) : 1;
+  for (rules.count = 0; rules.count < mla::CutRules::kMost; ++rules.count) {
+    mla::CutRules::Rule& r = rules.rule[rules.count];
+    const int rows = B > 0 ? mla::balanced_rows(B, R, block_size, tiles, nwg) : 0;
+    r.until = max_blocks > 0 || B == 0
+                  ? INT64_MAX
+                  : mla::balanced_rows_until(B, R, block_size, tiles, nwg);
+    r.nshare = rows > 0 ? wide_shares(n, R, rows, nwg) : n;
+    r.weight = rows > 0 ? mla::kWidePieceCost : 0;
+    if (r.until >= mla::kMaxTiles) break;
+    tiles = r.until + 1;
+  }
+  rules.rule[rules.count].until = INT64_MAX;
+  const int64_t cap = max_blocks > 0 ? (int64_t)max_blocks * block_size : INT32_MAX;
+  if (on_host) {
+    mla::host_num_splits(seq_lens, num_splits, B, block_size, cap, rules);
+    return hipSuccess;
+  }
+  hipLaunchKernelGGL(mla::mla_num_splits_kernel, dim3(1), dim3(mla::kNumSplitsThreads), 0, stream,
+                     seq_lens, num_splits, B, block_size, cap, rules);
+  return hipGetLastError();
 }
 
 extern "C" int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_cache,
@@ -1084,10 +1261,9 @@ extern "C" int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_
   a.nshare = n;
   const unsigned rg = (unsigned)((a.R + mla::kRowsPerGroup - 1) / mla::kRowsPerGroup);
   const int nwg = num_workgroups > 0 ? num_workgroups : gqa::device_cu_count();
-  const int rows = mla::wide_rows_balanced(a, nwg);
-  if (mla::wide_balanced(a, rows)) {
-    // (At most the n shares the workspace holds: rows <= 128.)
-    a.nshare = std::max(1, std::min(n, nwg / mla::row_groups(a.R, rows)));
+  const int rows = mla::balanced_rows(a.B, a.R, block_size, mla::tile_bound(a), nwg);
+  if (rows > 0) {
+    a.nshare = wide_shares(n, a.R, rows, nwg);
     a.piece_cost = mla::kWidePieceCost;
     if ((err = mla::launch_wide_balanced(a, rows, stream)) != hipSuccess) return err;
     return launch_balanced_merge(a, stream);

@@ -57,7 +57,7 @@ __device__ __forceinline__ int share_of(uint64_t U, uint64_t u, int n) {
 // 16.3 / 18.8 us. From about 2600 units on every CU has a share. As many shares
 // as requests cost no merge: 256 requests of 32 tokens, 16 heads, 14.5 us in 240
 // shares, 10.4 in 256.
-__device__ __forceinline__ int share_count(uint64_t U, int B, int nshare) {
+__host__ __device__ inline int share_count(uint64_t U, int B, int nshare) {
   uint64_t n = (uint64_t)(5.f * sqrtf((float)U)) + 1;
   n = n > (uint64_t)B ? n : (uint64_t)B;
   n = n < U ? n : U;

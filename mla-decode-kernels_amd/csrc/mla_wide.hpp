@@ -35,9 +35,7 @@ constexpr int kWidePieceCost = 8;
 // 16-token blocks, the gather -> here: one request of 4096 tokens, 128 heads,
 // 75.9 -> 20.0 us (its smaller row groups with it); 128 requests of ~4096
 // tokens 195.4 -> 179.1 (128 heads) and 144.0 -> 112.0 (16 heads).
-inline bool wide_blocks(const MlaArgs& a) {
-  return !MLA_PHASE_TIMING && a.block_size % 8 == 0;
-}
+inline bool wide_blocks(int block_size) { return !MLA_PHASE_TIMING && block_size % 8 == 0; }
 inline int64_t tile_bound(const MlaArgs& a) {  // tiles of the longest sequence
   return ((int64_t)a.max_blocks * a.block_size + kTile - 1) / kTile;
 }
@@ -69,14 +67,17 @@ inline int row_groups(int R, int rows) { return (R + rows - 1) / rows; }
 // rounds of smaller ones, unless every round of large ones is full: 256 of 200
 // (500), 128 heads, 45.4 -> 39.8, 43.3 (66.9 -> 63.0, 61.1) us, but 300 of 200
 // 60.4 -> 65.4. (256 of ~200, ragged, pay for it: 50.2 -> 54.2, 90.6.)
-inline int wide_rows_balanced(const MlaArgs& a, int nwg) {
-  const int64_t tiles = tile_bound(a), work = a.B * tiles * row_groups(a.R, 16);
-  int rows = wide_rows(a.R, work <= 12ll * nwg ? 16 : work <= 28ll * nwg ? 32
-                                                  : work <= 160ll * nwg ? 64 : 128);
-  const int most = wide_rows(a.R, 128);
-  if (tiles <= 2)
-    while (rows < most && (int64_t)a.B * row_groups(a.R, rows) > nwg) rows *= 2;
-  if (tiles >= 8 && (int64_t)a.B * row_groups(a.R, most) % nwg == 0) rows = most;
+constexpr int kWorkRows[3] = {12, 28, 160};  // most work of 16, 32 and 64 rows
+constexpr int kShortTiles = 2, kFullTiles = 8;
+inline int wide_rows_balanced(int B, int R, int64_t tiles, int nwg) {
+  const int64_t work = B * tiles * row_groups(R, 16);
+  int rows = 16;
+  for (int i = 0; i < 3 && work > (int64_t)kWorkRows[i] * nwg; ++i) rows *= 2;
+  rows = wide_rows(R, rows);
+  const int most = wide_rows(R, 128);
+  if (tiles <= kShortTiles)
+    while (rows < most && (int64_t)B * row_groups(R, rows) > nwg) rows *= 2;
+  if (tiles >= kFullTiles && (int64_t)B * row_groups(R, most) % nwg == 0) rows = most;
   return rows;
 }
 // Fixed splits: the largest row groups that still give every CU a workgroup.
@@ -97,11 +98,29 @@ inline int wide_rows_splitkv(const MlaArgs& a, int cus) {
 //    18.9 against 19.4 us; of 1024: 23.9 against 22.9), which only a caller
 //    that asks for a few workgroups brings to 128 rows.
 inline bool wide_splitkv(const MlaArgs& a, int rows) {
-  return wide_blocks(a) &&
+  return wide_blocks(a.block_size) &&
          (rows < 128 || a.num_splits == 1 || tile_bound(a) * kTile > 2048ll * a.num_splits);
 }
-inline bool wide_balanced(const MlaArgs& a, int rows) {
-  return wide_blocks(a) && (rows < 128 || a.B * tile_bound(a) > 8);
+constexpr int kFewTiles = 8;
+// Rows per workgroup of a balanced launch whose longest sequence has at most
+// `tiles` tiles, 0 for the 8-wave kernels.
+inline int balanced_rows(int B, int R, int block_size, int64_t tiles, int nwg) {
+  if (!wide_blocks(block_size)) return 0;
+  const int rows = wide_rows_balanced(B, R, tiles, nwg);
+  return rows < 128 || B * tiles > kFewTiles ? rows : 0;
+}
+// The most tiles, from `tiles` on, for which balanced_rows stays what it is.
+inline int64_t balanced_rows_until(int B, int R, int block_size, int64_t tiles, int nwg) {
+  const int64_t per_tile = (int64_t)B * row_groups(R, 16);
+  const int64_t ends[] = {kShortTiles, kFullTiles - 1, kFewTiles / B,
+                          (int64_t)kWorkRows[0] * nwg / per_tile,
+                          (int64_t)kWorkRows[1] * nwg / per_tile,
+                          (int64_t)kWorkRows[2] * nwg / per_tile};
+  const int rows = balanced_rows(B, R, block_size, tiles, nwg);
+  int64_t until = INT64_MAX;
+  for (const int64_t e : ends)
+    if (e >= tiles && e < until && balanced_rows(B, R, block_size, e + 1, nwg) != rows) until = e;
+  return until;
 }
 
 hipError_t launch_wide_splitkv(const MlaArgs& a, int rows, hipStream_t stream);

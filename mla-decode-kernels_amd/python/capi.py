@@ -94,6 +94,10 @@ def bind(path):
     L.mla_decode_combine_launch.argtypes = [_vp, ctypes.c_size_t, _vp, _vp, _i, _i, _i, _i,
                                             _vp]
     L.mla_decode_combine_launch.restype = _i
+    # (Builds of earlier sources, bound for comparison, lack it.)
+    if hasattr(L, "mla_decode_balanced_num_splits"):
+        L.mla_decode_balanced_num_splits.argtypes = [_vp, _vp] + [_i] * 7 + [_vp]
+        L.mla_decode_balanced_num_splits.restype = _i
     L.mla_decode_balanced_workspace_bytes.argtypes = [_i] * 4
     L.mla_decode_balanced_workspace_bytes.restype = ctypes.c_size_t
     L.mla_decode_workspace_bytes.argtypes = [_i] * 4
@@ -185,6 +189,10 @@ def mla_balanced_workspace_bytes(B, s_q, h_q, num_workgroups):
 
 def mla_workspace_bytes(B, s_q, h_q, num_splits):
     return lib().mla_decode_workspace_bytes(B, s_q, h_q, num_splits)
+
+
+def mla_balanced_num_splits(*args):
+    return lib().mla_decode_balanced_num_splits(*args)
 
 
 def mla_pick_num_splits(B, s_q, h_q, block_size, max_blocks, num_cus):

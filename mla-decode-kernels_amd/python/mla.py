@@ -47,9 +47,13 @@ def get_mla_metadata(cache_seqlens, num_heads_per_head_k, num_heads_k=1, max_seq
     [0, 0] = N > 0 selects N fixed splits per request. num_splits is, as in
     FlashMLA, the cumulative count of partial results per request ([b + 1]
     int32 on cache_seqlens' device), computed on the device for the balanced
-    plan. num_heads_per_head_k is s_q * h_q // h_kv; num_heads_k must be 1.
-    Passing num_splits=N asks for the fixed-split plan (max_seqlen bounds the
-    longest request for the split heuristic when N is 0)."""
+    plan: the launch's own cuts (mla_decode_balanced_num_splits) for a cache of
+    block_size tokens per block and a block table max_seqlen tokens wide, or as
+    wide as the longest request if max_seqlen is None. (The launch goes by the
+    width of the table it is given; a wider one can cut requests elsewhere.)
+    num_heads_per_head_k is s_q * h_q // h_kv; num_heads_k must be 1. Passing
+    num_splits=N asks for the fixed-split plan (max_seqlen bounds the longest
+    request for the split heuristic when N is 0)."""
     if num_heads_k != 1:
         raise ValueError("MLA decode supports one latent kv head (num_heads_k == 1)")
     if cache_seqlens.dtype != torch.int32 or cache_seqlens.dim() != 1:
@@ -70,25 +74,23 @@ def get_mla_metadata(cache_seqlens, num_heads_per_head_k, num_heads_k=1, max_seq
             raise ValueError("get_mla_metadata: invalid arguments")
         meta[0, 0] = ns
         return meta, torch.arange(b + 1, dtype=torch.int32, device=dev) * ns
-    rows = int(num_heads_per_head_k)
-    groups = max(1, -(-rows // 128))
     nwg = cus or 256
     meta[0, 1] = nwg
-    # Pieces per request with the request-ordered 32-token tiles cut into equal
-    # shares (share w of n: tiles [w T / n, (w + 1) T / n)). The launch plans
-    # for itself on the device and also weighs what a request costs besides its
-    # tiles, so it may cut a request once more or less than reported here.
-    n_share = max(1, nwg // groups)
-    tiles = (cache_seqlens.clamp(min=0).to(torch.int64) + 31) // 32
-    pre = torch.cumsum(tiles, 0)
-    p1, p0 = pre, pre - tiles
-    T = pre[-1:].clamp(min=1) if b else torch.ones(1, dtype=torch.int64, device=dev)
-    n = torch.minimum(torch.full_like(T, n_share), T)
-    w_lo = ((p0 + 1) * n - 1) // T
-    w_hi = (p1 * n - 1) // T
-    pieces = torch.where(tiles > 0, w_hi - w_lo + 1, torch.zeros_like(tiles))
-    splits = torch.zeros(b + 1, dtype=torch.int32, device=dev)
-    splits[1:] = torch.cumsum(pieces, 0).to(torch.int32)
+    splits = torch.empty(b + 1, dtype=torch.int32, device=dev)
+    lens = cache_seqlens.contiguous()
+    bs = max(1, int(block_size))
+    blocks = 0  # (a table as wide as the longest request)
+    if max_seqlen is not None:
+        blocks = min(max(1, -(-int(max_seqlen) // bs)), ((1 << 31) - 1) // bs)
+    args = (lens.data_ptr(), splits.data_ptr(), b, 1,
+            min(max(1, int(num_heads_per_head_k)), 1 << 20), bs, blocks, nwg)
+    if dev.type == "cuda":
+        with torch.cuda.device(dev):
+            rc = capi.mla_balanced_num_splits(*args, 0, torch.cuda.current_stream(dev).cuda_stream)
+    else:
+        rc = capi.mla_balanced_num_splits(*args, 1, None)
+    if rc != 0:
+        raise RuntimeError(f"get_mla_metadata: HIP error {rc}")
     return meta, splits
 
 

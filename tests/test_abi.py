@@ -408,7 +408,8 @@ def test_op_check_order_and_messages(binding):
 
 def test_mla_exports():
     declared = capi.declared_mla_functions()
-    assert declared == ["mla_decode_balanced_launch", "mla_decode_balanced_workspace_bytes",
+    assert declared == ["mla_decode_balanced_launch", "mla_decode_balanced_num_splits",
+                        "mla_decode_balanced_workspace_bytes",
                         "mla_decode_combine_launch", "mla_decode_launch",
                         "mla_decode_pick_num_splits", "mla_decode_splitkv_launch",
                         "mla_decode_workspace_bytes"]
