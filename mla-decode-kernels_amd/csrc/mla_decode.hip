@@ -883,7 +883,7 @@ __global__ __launch_bounds__(64 * NW) void mla_decode_balanced_merge_kernel(cons
 
 // The launch's row groups by the tiles of the longest sequence.
 struct CutRules {
-  static constexpr int kMost = 8;  // (balanced_rows changes at six places at most)
+  static constexpr int kMost = 8;  // (balanced_rows changes at five places at most)
   struct Rule {
     int64_t until;  // up to this many tiles
     int nshare, weight;
@@ -1268,10 +1268,12 @@ extern "C" int mla_decode_balanced_launch(const uint16_t* q, const uint16_t* kv_
     if ((err = mla::launch_wide_balanced(a, rows, stream)) != hipSuccess) return err;
     return launch_balanced_merge(a, stream);
   }
+#if MLA_PHASE_TIMING
   if (block_size % mla::kTile == 0)
     hipLaunchKernelGGL(mla::mla_decode_balanced_kernel<true>, dim3(n, rg), dim3(mla::kThreads), 0,
                        stream, a);
   else
+#endif
     hipLaunchKernelGGL(mla::mla_decode_balanced_kernel<false>, dim3(n, rg), dim3(mla::kThreads), 0,
                        stream, a);
   if ((err = hipGetLastError()) != hipSuccess) return err;

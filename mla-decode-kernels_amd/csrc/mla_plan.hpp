@@ -49,13 +49,17 @@ __device__ __forceinline__ int share_of(uint64_t U, uint64_t u, int n) {
 }
 
 // Shares for U units of B requests: at most nshare, and no more than 5 sqrt(U)
-// or one per request. A share costs
-// its units one after the other (~1.5 us each) and its states in the merge
-// (~0.06 us per share for 128 rows), so with little work fewer shares than CUs
-// are faster. One request of 4096 tokens, 128 heads (136 units): 36.8 / 31.6 /
-// 28.8 / 31.0 us at 136 / 68 / 34 / 17 shares; 16 heads (132): 17.7 / 15.7 /
-// 16.3 / 18.8 us. From about 2600 units on every CU has a share. As many shares
-// as requests cost no merge: 256 requests of 32 tokens, 16 heads, 14.5 us in 240
+// or one per request. A share costs its units one after the other and its states
+// in the merge, so with little work fewer shares than CUs can be faster. Balanced
+// launch (us) with at most 2.5 / 5 / 10 sqrt(U) shares and one per CU, 16 heads:
+//   1 request of 4096 tokens    16.6   15.6   17.1   17.2
+//   1 of 1000                   14.2   13.6   13.1   13.1
+//   1 of 16384                  21.1   20.7   24.6   24.4
+//   3 of ~16384, 32 heads       29.5   28.1   30.4   30.5
+//   16 of ~500                  18.5   16.4   16.1   16.6
+// (At more heads the row groups often leave fewer shares than that: one request
+// of 1000 tokens, 128 heads, 15.6 / 16.6 / 16.6 / 16.6.) As many shares as
+// requests cost no merge: 256 requests of 32 tokens, 16 heads, 14.5 us in 240
 // shares, 10.4 in 256.
 __host__ __device__ inline int share_count(uint64_t U, int B, int nshare) {
   uint64_t n = (uint64_t)(5.f * sqrtf((float)U)) + 1;

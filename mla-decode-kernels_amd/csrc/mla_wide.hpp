@@ -89,30 +89,25 @@ inline int wide_rows_splitkv(const MlaArgs& a, int cus) {
 }
 
 // Whether the wide kernels run. At 128 rows per workgroup the 8-wave kernels
-// keep
-//  - fixed splits (num_splits > 1) of at most 2048 tokens of the longest
-//    sequence: twice the waves load Q and store the states, which weighs more
-//    than the tiles there (64 requests of ~1024 tokens at 4 splits, 128 rows:
-//    51.8 against 55.5 us; of ~4096 tokens: 124.6 against 121.3);
-//  - balanced launches of at most 8 tiles in all (one request of 64 tokens:
-//    18.9 against 19.4 us; of 1024: 23.9 against 22.9), which only a caller
-//    that asks for a few workgroups brings to 128 rows.
+// keep fixed splits (num_splits > 1) of at most 2048 tokens of the longest
+// sequence: twice the waves load Q and store the states, which weighs more than
+// the tiles there (64 requests of ~1024 tokens at 4 splits, 128 rows: 51.8
+// against 55.5 us; of ~4096 tokens: 124.6 against 121.3).
 inline bool wide_splitkv(const MlaArgs& a, int rows) {
   return wide_blocks(a.block_size) &&
          (rows < 128 || a.num_splits == 1 || tile_bound(a) * kTile > 2048ll * a.num_splits);
 }
-constexpr int kFewTiles = 8;
 // Rows per workgroup of a balanced launch whose longest sequence has at most
-// `tiles` tiles, 0 for the 8-wave kernels.
+// `tiles` tiles, 0 for the 8-wave kernels (they run the other block sizes alone:
+// on few workgroups and tiles too they are slower, 512 rows of one request on
+// one of 128 rows, 64 tokens 20.9 against 18.2 us, 256 tokens 29.1 against 26.2).
 inline int balanced_rows(int B, int R, int block_size, int64_t tiles, int nwg) {
-  if (!wide_blocks(block_size)) return 0;
-  const int rows = wide_rows_balanced(B, R, tiles, nwg);
-  return rows < 128 || B * tiles > kFewTiles ? rows : 0;
+  return wide_blocks(block_size) ? wide_rows_balanced(B, R, tiles, nwg) : 0;
 }
 // The most tiles, from `tiles` on, for which balanced_rows stays what it is.
 inline int64_t balanced_rows_until(int B, int R, int block_size, int64_t tiles, int nwg) {
   const int64_t per_tile = (int64_t)B * row_groups(R, 16);
-  const int64_t ends[] = {kShortTiles, kFullTiles - 1, kFewTiles / B,
+  const int64_t ends[] = {kShortTiles, kFullTiles - 1,
                           (int64_t)kWorkRows[0] * nwg / per_tile,
                           (int64_t)kWorkRows[1] * nwg / per_tile,
                           (int64_t)kWorkRows[2] * nwg / per_tile};

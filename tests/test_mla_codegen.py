@@ -92,7 +92,6 @@ def tile_loops(body):
 
 KERNELS = ["_ZN3mla17mla_decode_kernelILb1EEEvNS_7MlaArgsE",
            "_ZN3mla17mla_decode_kernelILb0EEEvNS_7MlaArgsE",
-           "_ZN3mla26mla_decode_balanced_kernelILb1EEEvNS_7MlaArgsE",
            "_ZN3mla26mla_decode_balanced_kernelILb0EEEvNS_7MlaArgsE"]
 
 

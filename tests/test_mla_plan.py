@@ -35,7 +35,7 @@ def row_groups(B, rows, block_size, width, nwg):
         r = next((x for x in sizes if x >= r and B * groups(x) <= nwg), sizes[-1])
     if tiles >= 8 and B * groups(sizes[-1]) % nwg == 0:
         r = sizes[-1]
-    return (groups(r), WEIGHT) if r < 128 or B * tiles > 8 else (groups(128), 0)
+    return groups(r), WEIGHT
 
 
 def simulate(S_list, rows, block_size, longest, nwg):
