@@ -4,9 +4,13 @@ the oracle at the sizes where they can go wrong -- row counts around the 16, 32,
 ring holds four), shares of many short pieces, second passes in the middle of a
 share -- and CPU checks of the generated code.
 
-Tolerance (that of test_mla.py): weights are rounded to bf16 for the PV product
-and the output to bf16, each within 2^-9 relative, so |out - oracle| is at most
-2^-8 of the largest value row entry (~4.5 for N(0, 1)): 1.8e-2.
+Tolerance, element by element (that of test_mla.py): weights are rounded to bf16
+for the PV product and the output to bf16, each within 2^-9 relative, so |out -
+oracle| is at most 2^-8 of the largest value row entry (~4.5 for N(0, 1)):
+1.8e-2. That is more than a whole output of many tokens, so each row's error is
+also held against the row, 2-norm over 2-norm: independent value rows add the
+weights' errors in squares, 2^-9 of the row, and the output's rounding another
+2^-9; 1e-2 leaves a factor of 2.5 for value rows that are not.
 """
 
 import os
@@ -20,8 +24,44 @@ import torch
 
 import capi
 from cases import make_mla_case
-from test_mla import SCALE, check, oracle, run, run_balanced
+from test_mla import SCALE, oracle, run, run_balanced
+from test_mla import check as check_elements
 from test_mla_codegen import HIPCC, ROOT, kernel_body, tile_loops
+
+ROW_REL = 1e-2
+
+
+def row_errors(out, want):
+    """2-norm of each row's error over that of the row (0 for rows of zeros)."""
+    off, size = np.linalg.norm(out - want, axis=-1), np.linalg.norm(want, axis=-1)
+    return np.where(size > 0, off / np.where(size > 0, size, 1.0), off)
+
+
+def check(got, want, label):
+    check_elements(got, want, label)
+    worst = float(row_errors(got[0].float().cpu().numpy(), want[0]).max())
+    assert worst <= ROW_REL, f"{label}: a row is {worst:.1e} off"
+
+
+@pytest.mark.parametrize("S,pieces", [(300, 4), (4096, 59), (9000, 64)])
+def test_check_sees_a_lost_tile(S, pieces):
+    # What the element-wise tolerance lets pass in long requests: a kernel that
+    # leaves a tile out of the PV product, takes the last tile's weights for it,
+    # or loses the accumulator of one piece while keeping its sum of weights.
+    rng = np.random.default_rng(S)
+    q, keys = rng.standard_normal((8, 576)), rng.standard_normal((S, 576))
+    p = np.exp(q @ keys.T * SCALE)
+    p /= p.sum(axis=1, keepdims=True)
+    want = p @ keys[:, :512]
+    at = 32 * (S // 64)
+    lost, stale, piece = p.copy(), p.copy(), p.copy()
+    lost[:, at:at + 32] = 0
+    stale[:, at:at + 32] = p[:, at - 32:at]
+    piece[:, at:at + S // pieces] = 0
+    for wrong in (lost, stale, piece):
+        assert row_errors(wrong @ keys[:, :512], want).max() > 2 * ROW_REL
+    assert row_errors(want.astype(np.float32), want).max() < 1e-6
+
 
 EDGES = [1, 31, 32, 33, 0, 63, 64, 65, 95, 96, 97, 128, 129, 161, 300]
 # (s_q, h_q): one row; the 16-, 32-, 64- and 128-row variants, full and one
@@ -116,6 +156,26 @@ def test_few_tiles_on_few_workgroups(gpu, S_list, s_q, nwg):
         check(run_balanced(case, causal, nwg), oracle(case, causal), f"{S_list}/n{nwg}/c{causal}")
     pre, n = launched_plan(case, nwg)
     assert n == 1 and pre[1] == -(-S_list[0] // 32) + 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h_q,nwg", [(16, 256), (32, 256), (128, 256), (128, 60), (128, 12),
+                                     (128, 2)])
+@pytest.mark.parametrize("S_list", [[5, 100, 33], [2100, 700, 64]])
+def test_lse_accuracy(gpu, h_q, nwg, S_list):
+    # lse sums the weights before their rounding: the largest error here is that
+    # of a few fp32 roundings near the value (|lse| < 16: an ulp is 2^-20), where
+    # rounded weights are 1e-5 to 1e-3 off. In every row variant, direct and
+    # merged.
+    case = make_mla_case(S_list, 1, h_q, 64, pool_factor=1.5, seed=h_q, device="cuda", poison=True)
+    q, kv, bt, _ = case
+    _, lse = run_balanced(case, False, nwg)
+    for b, S in enumerate(S_list):
+        keys = kv[bt[b, :-(-S // 64)].long()].flatten(0, 1)[:S, 0].double()
+        exact = torch.logsumexp(torch.matmul(q[b, 0].double(), keys.t().contiguous()) * SCALE, 1)
+        assert float(exact.abs().max()) < 16
+        off = float((lse[b, :, 0].double() - exact).abs().max())
+        assert off <= 6 * 2.0 ** -20, f"S={S}: {off:.1e} off"
 
 
 @pytest.mark.gpu
