@@ -592,19 +592,21 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
     const bool direct = uniform((int)po.direct) != 0;
     if (row0 < a.R) {
       const float L = Sh::row_sum(lsum), Lpv = Sh::row_sum(lpv);
-      // out = o / Lpv; a state's rows, normalised by its L later on, o L / Lpv.
-      const float factor = L > 0.f ? (direct ? 1.f : L) / Lpv : direct ? 0.f : 1.f;
+      const float inv = L > 0.f ? 1.f / Lpv : 0.f;
       const int l = fresh_lane();
       const int row = row0 + l % RW;
       if (row < a.R && l < RW && part == 0) {
+        // lse; or a state's m (natural-log units), for a sum of Lpv, what its
+        // rows are a weighted sum by: m + ln Lpv is the piece's lse. (Rows scaled
+        // to a sum of L instead cost 0.1 to 0.2 us of a call.)
+        const float x = L > 0.f ? logf(direct ? L : L * inv) - nbase * kLn2 : kNegInf;
         if (!direct) {
           const size_t sx = po.st_base + (size_t)row * po.st_stride;
-          a.ws_m[sx] = L > 0.f ? -nbase * kLn2 : kNegInf;  // natural-log units
-          a.ws_l[sx] = L;
+          a.ws_m[sx] = x;
+          a.ws_l[sx] = Lpv;
         } else if (a.lse) {
           const int qi = row / a.h_q, hq = row - qi * a.h_q;
-          a.lse[((size_t)p.b * a.h_q + hq) * a.s_q + qi] =
-              L > 0.f ? logf(L) - nbase * kLn2 : kNegInf;
+          a.lse[((size_t)p.b * a.h_q + hq) * a.s_q + qi] = x;
         }
       }
       const uint32_t buf =
@@ -612,12 +614,12 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
       const uint32_t dst = buf + (uint32_t)(l % RW) * 256;
       // This lane's rows 4 i + l / 16: what it reads back and stores. (Past the
       // last row: the last row's values once more.)
-      float fr[RW / 4];
+      float iv[RW / 4];
       uint32_t off[RW / 4];
 #pragma unroll
       for (int i = 0; i < RW / 4; ++i) {
         const int r = 4 * i + (l >> 4);
-        fr[i] = __shfl(factor, r, 64);
+        iv[i] = __shfl(inv, r, 64);
         off[i] = (uint32_t)min(r, a.R - 1 - row0);
       }
       const int dim0 = part * (kDV / kParts) + 4 * (l & 15);
@@ -647,14 +649,12 @@ __device__ __forceinline__ void wide_run(const MlaArgs& a, uint8_t* smem, int rg
 #pragma unroll
           for (int i = 0; i < RW / 4; ++i)
             *reinterpret_cast<uint2*>(out0 + off[i] * kDV + 64 * k) =
-                make_uint2(pack_bf16(__uint_as_float(v[i].x) * fr[i], __uint_as_float(v[i].y) * fr[i]),
-                           pack_bf16(__uint_as_float(v[i].z) * fr[i], __uint_as_float(v[i].w) * fr[i]));
+                make_uint2(pack_bf16(__uint_as_float(v[i].x) * iv[i], __uint_as_float(v[i].y) * iv[i]),
+                           pack_bf16(__uint_as_float(v[i].z) * iv[i], __uint_as_float(v[i].w) * iv[i]));
         } else {
 #pragma unroll
           for (int i = 0; i < RW / 4; ++i)
-            *reinterpret_cast<float4*>(acc0 + off[i] * pitch + 64 * k) =
-                make_float4(__uint_as_float(v[i].x) * fr[i], __uint_as_float(v[i].y) * fr[i],
-                            __uint_as_float(v[i].z) * fr[i], __uint_as_float(v[i].w) * fr[i]);
+            *reinterpret_cast<u32x4_t*>(acc0 + off[i] * pitch + 64 * k) = v[i];
         }
       }
     }
