@@ -518,7 +518,7 @@ def main_mla(args, dev, props):
         "pct_of_sol": round(sol / median_us * 100, 2),
         "flashmla_h100_us": h100 * 1e3 if h100 else None,
         "roofline": {"bound": bound,
-                     "kernel": "whole step" if balanced else "mla_decode_kernel",
+                     "kernel": "whole step" if balanced else "split kernel",
                      "achieved": round(achieved, 1),
                      "peak": peak, "unit": "TFLOP/s" if bound == "mfma" else "GB/s",
                      "frac": round(achieved / peak, 4), "avg_kernel_us": round(kern_us, 3),

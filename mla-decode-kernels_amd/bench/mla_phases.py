@@ -1,5 +1,8 @@
-"""Where the MLA decode's waves spend their cycles: the phase table of a
-profiling build of the kernel library.
+"""Where the waves of the 8-wave MLA kernels spend their cycles: the phase table
+of a profiling build of the kernel library, which runs those kernels for every
+call. (The shipped library runs them for block sizes off 8 and for short fixed
+splits of 128 rows; the balanced launch of the benchmark rows takes the
+one-wave-per-SIMD kernels, which have no stamps.)
 
     python mla-decode-kernels_amd/build.py --variant phase --define MLA_PHASE_TIMING=1
     python mla-decode-kernels_amd/bench/mla_phases.py --config mla_4k
